@@ -216,25 +216,58 @@ __global__ void gelu_back_kernel(int M, int N, const float* __restrict__ parts, 
   }
 }
 
-// out[n] = sum_m x[m][n]
-__global__ void colsum_kernel(int M, int N, const float* __restrict__ x, float* __restrict__ out) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
+// out[n] = sum_m x[m][n].  A workgroup takes 64 columns; its 16 waves share the rows (wave w:
+// rows w, w + 16, ...) and their partial sums are added in wave order.  One thread per column
+// over all rows was a chain of M dependent loads on 29 workgroups and fewer: 56.9 us on average over a
+// training step's three (256 x 7200, which is 7.4 MB, and twice 256 x 512); this form 4.3 us.
+constexpr int CSW = 16;
+__global__ __launch_bounds__(64 * CSW) void colsum_kernel(int M, int N, const float* __restrict__ x,
+                                                          float* __restrict__ out) {
+  __shared__ float sh[CSW][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n = blockIdx.x * 64 + lane;
   float s = 0.f;
-  for (int m = 0; m < M; ++m) s += x[(long long)m * N + n];
-  out[n] = s;
+  if (n < N) {
+#pragma unroll 8
+    for (int m = wave; m < M; m += CSW) s += x[(long long)m * N + n];
+  }
+  sh[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && n < N) {
+    for (int w = 1; w < CSW; ++w) s += sh[w][lane];
+    out[n] = s;
+  }
 }
 
-// out[c][n] = sum over rows m of channel c of x[m][n]
-__global__ void embgrad_kernel(int M, int N, int nchan, const float* __restrict__ x, const int* __restrict__ chan,
-                               float* __restrict__ out) {
-  const long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (idx >= (long long)nchan * N) return;
-  const int c = (int)(idx / N), n = (int)(idx % N);
+// out[c][n] = sum over rows m of channel c of x[m][n], in increasing m.  One wave per (64
+// columns, channel): a ballot over 64 rows' channels gives the rows of c, whose values are
+// loaded four at a time.  With a thread per (c, n) walking all rows the loop's branch per row
+// cost 18.5 us at 256 rows x 512 columns x 42 channels; this form 3.5 us.
+__global__ __launch_bounds__(64) void embgrad_kernel(int M, int N, const float* __restrict__ x,
+                                                     const int* __restrict__ chan, float* __restrict__ out) {
+  const int strips = (N + 63) / 64;
+  const int c = blockIdx.x / strips, lane = threadIdx.x;
+  const int n = (blockIdx.x - c * strips) * 64 + lane;
+  const float* xn = x + min(n, N - 1);
   float s = 0.f;
-  for (int m = 0; m < M; ++m)
-    if (chan[m] == c) s += x[(long long)m * N + n];
-  out[idx] = s;
+  for (int m0 = 0; m0 < M; m0 += 64) {
+    unsigned long long rows = __ballot(m0 + lane < M && chan[min(m0 + lane, M - 1)] == c);
+    while (rows) {
+      float v[4];
+      bool on[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        on[q] = rows != 0;
+        const int m = on[q] ? m0 + __builtin_ctzll(rows) : m0;
+        rows &= rows - 1;  // stays 0 once empty
+        v[q] = xn[(long long)m * N];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (on[q]) s += v[q];
+    }
+  }
+  if (n < N) out[(long long)c * N + n] = s;
 }
 
 __global__ void to_bf16_kernel(long long n, const float* __restrict__ x, uint16_t* __restrict__ y) {
@@ -371,13 +404,13 @@ double Learned::backward(int rows, const int* chan, const float* t, hipStream_t 
                      loss_part.ptr);
   // layer 3
   gemm_bf16(in, hidden, rows, gh.ptr, 1, in, h2h.ptr, hidden, 1, grads.ptr + o_w3, 1, s);
-  hipLaunchKernelGGL(colsum_kernel, dim3((in + 255) / 256), dim3(256), 0, s, rows, in, gf.ptr, grads.ptr + o_b3);
+  hipLaunchKernelGGL(colsum_kernel, dim3(ceil_div(in, 64)), dim3(64 * CSW), 0, s, rows, in, gf.ptr, grads.ptr + o_b3);
   int sp = gemm_bf16(rows, hidden, in, gh.ptr, in, 1, w3h.ptr, hidden, 1, part.ptr,
                      std::min(splits_max, pick_splits(rows, hidden, in)), s);
   hipLaunchKernelGGL(gelu_back_kernel, dim3(grid_for_n(rh)), dim3(256), 0, s, rows, hidden, part.ptr, sp, z2.ptr,
                      dzf.ptr, dz2h.ptr);
   // layer 2
-  hipLaunchKernelGGL(colsum_kernel, dim3((hidden + 255) / 256), dim3(256), 0, s, rows, hidden, dzf.ptr,
+  hipLaunchKernelGGL(colsum_kernel, dim3(ceil_div(hidden, 64)), dim3(64 * CSW), 0, s, rows, hidden, dzf.ptr,
                      grads.ptr + o_b2);
   gemm_bf16(hidden, hidden, rows, dz2h.ptr, 1, hidden, h1h.ptr, hidden, 1, grads.ptr + o_w2, 1, s);
   sp = gemm_bf16(rows, hidden, hidden, dz2h.ptr, hidden, 1, w2h.ptr, hidden, 1, part.ptr,
@@ -385,10 +418,10 @@ double Learned::backward(int rows, const int* chan, const float* t, hipStream_t 
   hipLaunchKernelGGL(gelu_back_kernel, dim3(grid_for_n(rh)), dim3(256), 0, s, rows, hidden, part.ptr, sp, z1.ptr,
                      dzf.ptr, dz1h.ptr);
   // layer 1
-  hipLaunchKernelGGL(colsum_kernel, dim3((hidden + 255) / 256), dim3(256), 0, s, rows, hidden, dzf.ptr,
+  hipLaunchKernelGGL(colsum_kernel, dim3(ceil_div(hidden, 64)), dim3(64 * CSW), 0, s, rows, hidden, dzf.ptr,
                      grads.ptr + o_b1);
-  hipLaunchKernelGGL(embgrad_kernel, dim3((int)ceil_div((long long)nchan * hidden, 256)), dim3(256), 0, s, rows,
-                     hidden, nchan, dzf.ptr, chan, grads.ptr + o_emb);
+  hipLaunchKernelGGL(embgrad_kernel, dim3(ceil_div(hidden, 64) * nchan), dim3(64), 0, s, rows, hidden, dzf.ptr, chan,
+                     grads.ptr + o_emb);
   gemm_bf16(hidden, in, rows, dz1h.ptr, 1, hidden, xh.ptr, in, 1, grads.ptr + o_w1, 1, s);
   PP_HIP(hipGetLastError());
   if (!want_loss) return 0.0;

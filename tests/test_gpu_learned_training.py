@@ -1,0 +1,70 @@
+"""GPU tests of the training kernels of the learned preconditioner at the edges of their tiles
+(rows, hidden width and channels that are no multiple of a wave) against the float64 oracle
+with the device's BF16 rounding points."""
+import numpy as np
+import pytest
+
+from oracle import mlp
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+    assert t.cuda.is_available(), "GPU tests need a HIP device"
+    from pyprop_amd import _native
+    _native.load()
+    return t
+
+
+class _Shape:
+    def __init__(self, nchan, n):
+        self.system = type("System", (), {"shape": (nchan, n, n)})
+
+    def Setup(self):
+        pass
+
+
+def _rel(a, b):
+    return np.linalg.norm(np.ravel(a) - np.ravel(b)) / max(np.linalg.norm(np.ravel(b)), 1e-300)
+
+
+def _case(nchan, n, hidden, rows, seed):
+    from pyprop_amd.mixed import LearnedPreconditioner
+    rng = np.random.default_rng(seed)
+    net = LearnedPreconditioner(_Shape(nchan, n), hidden)
+    inp = 2 * n * n
+    flat = net.get_params().astype(np.float64)
+    lay, _ = mlp.layout(inp, hidden, nchan)
+    for name, scale in (("W3", hidden ** -0.5), ("b1", 0.1), ("emb", 0.1), ("b2", 0.1), ("b3", 0.1)):
+        o, shp = lay[name]
+        k = int(np.prod(shp))
+        flat[o:o + k] = scale * rng.standard_normal(k)
+    flat = flat.astype(np.float32)
+    net.set_params(flat)
+    x = (rng.standard_normal((rows, inp)) / np.sqrt(inp)).astype(np.float32)
+    t = (0.3 * rng.standard_normal((rows, inp))).astype(np.float32)
+    chan = rng.integers(0, nchan, rows).astype(np.int32)
+    return net, flat, x, t, chan
+
+
+# rows below, at and above a ballot of 64 and the 16 waves of a column sum; widths below and
+# above the 64 columns of a workgroup; channels without a row
+@pytest.mark.parametrize("dims", [(1, 1, 8, 1), (5, 3, 72, 15), (70, 2, 64, 64), (9, 6, 136, 65), (2, 5, 64, 203)],
+                         ids=lambda d: "x".join(map(str, d)))
+def test_gradients_at_tile_edges(torch, dims):
+    nchan, n, hidden, rows = dims
+    net, flat, x, t, chan = _case(nchan, n, hidden, rows, 3)
+    inp = 2 * n * n
+    dev = [torch.from_numpy(a).to("cuda") for a in (x, chan, t)]
+    loss = net.gradient(*dev)
+    loss_ref, g_ref = mlp.loss_and_grad(mlp.unpack(flat.astype(np.float64), inp, hidden, nchan), x, chan, t, 1.0)
+    assert abs(loss - loss_ref) < 1e-4 * loss_ref
+    g = mlp.unpack(net.get_grads().astype(np.float64), inp, hidden, nchan)
+    for name in mlp.NAMES:
+        # FP32 sums; a backward signal whose FP32 value sits on a BF16 rounding boundary moves
+        # by one BF16 ulp (2^-8), which few of a sum's terms do
+        assert _rel(g[name], g_ref[name]) < 2e-3, name
+    for c in set(range(nchan)) - set(chan.tolist()):
+        assert np.all(g["emb"][c] == 0)
