@@ -44,51 +44,120 @@ __device__ inline float gelu_grad(float z) {
   return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// 16 bytes at byte offset off of the buffer behind r (range-checked: zeros past its end, so a
+// masked-out lane passes kOff16 and its load needs no branch)
+constexpr int kOff16 = 0x7ffffff0;  // beyond every buffer read this way (all under 2 GiB)
+__device__ __forceinline__ u32x4 ld16(__amdgpu_buffer_rsrc_t r, int off) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, long long bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+}
+
 static int grid_for_n(long long n) {
   long long b = (n + 255) / 256;
   return (int)std::max(1LL, std::min(b, 4096LL));
 }
 
 // ------------------------------------------------------------------------------------
-// BF16 GEMM on MFMA: 64 x 64 tile per workgroup, four waves of 32 x 32, K step 32
+// BF16 GEMM on MFMA: 64 x 64 tile per workgroup, four waves of 32 x 32, K step 64
 // ------------------------------------------------------------------------------------
-constexpr int GBM = 64, GBN = 64, GBK = 32, GLD = GBK + 8;  // LDS row: 40 BF16 = 80 B
+// The products here are small (256 x 512 x 7200 and its transposes): each workgroup runs 4 to 16
+// K steps, so what bounds it is the latency of a step, not the matrix cores.  A step's operands
+// are therefore loaded into registers two steps ahead (the loads of a whole step, 16 bytes each,
+// in flight together) and stored into the other of two LDS buffers while the matrix cores work
+// from the first: one barrier per step.
+// LDS holds X(r, k) as 64 rows of 64 BF16 without padding; the 16-byte chunk c of row r sits at
+// c ^ (r ^ r >> 3) & 7, so that the 16 rows of an operand read and the rows that a transposed
+// store touches fall in different banks.  An operand stored with k as the slow index is
+// transposed on the way: a thread loads the same 8 rows at k and k + 1 and stores 8 (k, k + 1)
+// pairs.
+// One K step of 32 at a time, loaded, stored and used in turn: 17.8 us per product over a training
+// step's eight (256 rows, 7200 -> 512 -> 512 -> 7200); this form 8.0 us (the four long ones 17 -> 8.7 to
+// 11.2, of which the 14.7 MB of FP32 gradients written take 3).  Loads behind a branch on the tile edge
+// made the compiler wait for all of them at each step: 11.1 us.
+constexpr int GBM = 64, GBN = 64, GBK = 64;
 
-// Tile rows r0..r0+63, k0..k0+31 of X(r, k) = p[r*sr + k*sk] into S[r][k] (zero padded).
-__device__ inline void load_tile(const uint16_t* __restrict__ p, long long sr, long long sk, int R, int r0, int k0,
-                                 int ke, uint16_t* S, int t) {
-  if (sk == 1) {
-    const int r = t >> 2, kk = (t & 3) * 8;
-    const int gr = r0 + r, gk = k0 + kk;
-    if (gr < R && gk + 8 <= ke && (sr & 7) == 0) {
-      *reinterpret_cast<uint4*>(&S[r * GLD + kk]) = *reinterpret_cast<const uint4*>(p + (long long)gr * sr + gk);
+__device__ __forceinline__ int gswz(int r, int chunk) { return (chunk ^ r ^ (r >> 3)) & 7; }
+
+struct GemmFrag {
+  u32x4 v[2];
+};
+
+// Thread t's share of the tile rows r0..r0+63, k0..k0+63 of X(r, k) = p[r*sr + k*sk], zeros outside.
+// KC (k contiguous): rows t / 8 and t / 8 + 32, k chunk t % 8.  Otherwise rows 8 (t % 8) .. + 7 at
+// k = 2 (t / 8) and the next.  WIDE (see gemm_wide): 16-byte range-checked loads, a share outside
+// the operand past the range, so that no load waits at a branch.
+template <bool KC, bool WIDE>
+__device__ __forceinline__ GemmFrag gemm_load(const uint16_t* __restrict__ p, long long sr, long long sk, int R, int r0,
+                                              int k0, int ke, int t) {
+  GemmFrag f;
+  const __amdgpu_buffer_rsrc_t tile = rsrc(p + (KC ? (long long)r0 * sr : (long long)r0), kOff16 - 16);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = KC ? r0 + (t >> 3) + 32 * h : r0 + (t & 7) * 8;
+    const int k = KC ? k0 + (t & 7) * 8 : k0 + (t >> 3) * 2 + h;
+    if (WIDE) {
+      const int off = KC ? ((r - r0) * (int)sr + k) * 2 : (k * (int)sk + (r - r0)) * 2;
+      f.v[h] = ld16(tile, r < R && k < ke ? off : kOff16);
     } else {
 #pragma unroll
-      for (int q = 0; q < 8; ++q)
-        S[r * GLD + kk + q] = (gr < R && gk + q < ke) ? p[(long long)gr * sr + gk + q] : (uint16_t)0;
+      for (int q = 0; q < 4; ++q) {
+        unsigned w[2] = {0, 0};
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int rr = KC ? r : r + 2 * q + e, kk = KC ? k + 2 * q + e : k;
+          if (rr < R && kk < ke) w[e] = p[(long long)rr * sr + (long long)kk * sk];
+        }
+        f.v[h][q] = w[0] | (w[1] << 16);
+      }
+    }
+  }
+  return f;
+}
+
+// Whether an operand of R rows (k in [0, K)) can be read 16 bytes at a time: shares of eight lie
+// inside or outside it as a whole and are 16-byte aligned, and a tile's offsets fit the 31 bits of
+// a buffer offset.
+static bool gemm_wide(const uint16_t* p, int R, int K, long long sr, long long sk) {
+  if (reinterpret_cast<uintptr_t>(p) & 15) return false;
+  if (sk == 1) return sr % 8 == 0 && K % 8 == 0 && sr >= 0 && 2 * (GBM * sr + K) < kOff16 - 16;
+  return sr == 1 && sk % 8 == 0 && R % 8 == 0 && sk >= 0 && 2 * (K * sk + GBM) < kOff16 - 16;
+}
+
+template <bool KC>
+__device__ __forceinline__ void gemm_store(const GemmFrag& f, uint16_t* S, int t) {
+  if (KC) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int r = (t >> 3) + 32 * h;
+      *reinterpret_cast<u32x4*>(&S[r * GBK + gswz(r, t & 7) * 8]) = f.v[h];
     }
   } else {
-    const int kk = t >> 3, rr = (t & 7) * 8;
-    const int gk = k0 + kk, gr = r0 + rr;
-    if (gk < ke && gr + 8 <= R && sr == 1 && (sk & 7) == 0) {
-      const uint4 q4 = *reinterpret_cast<const uint4*>(p + (long long)gk * sk + gr);
-      const uint16_t* v = reinterpret_cast<const uint16_t*>(&q4);
+    const int k = (t >> 3) * 2;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) S[(rr + q) * GLD + kk] = v[q];
-    } else {
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        S[(rr + q) * GLD + kk] = (gk < ke && gr + q < R) ? p[(long long)(gr + q) * sr + (long long)gk * sk] : (uint16_t)0;
+    for (int q = 0; q < 8; ++q) {
+      const int r = (t & 7) * 8 + q;
+      const unsigned lo = (q & 1) ? f.v[0][q >> 1] >> 16 : f.v[0][q >> 1] & 0xFFFFu;
+      const unsigned hi = (q & 1) ? f.v[1][q >> 1] & 0xFFFF0000u : f.v[1][q >> 1] << 16;
+      *reinterpret_cast<unsigned*>(&S[r * GBK + gswz(r, k >> 3) * 8 + (k & 7)]) = lo | hi;
     }
   }
 }
 
+template <bool AK, bool BK, bool WIDE>
 __global__ __launch_bounds__(256) void gemm_bf16_kernel(int M, int N, int K, int kchunk, const uint16_t* __restrict__ a,
                                                         long long sam, long long sak, const uint16_t* __restrict__ b,
                                                         long long sbk, long long sbn, float* __restrict__ c) {
-  __shared__ __align__(16) uint16_t As[GBM * GLD];
-  __shared__ __align__(16) uint16_t Bs[GBN * GLD];
-  const int m0 = blockIdx.y * GBM, n0 = blockIdx.x * GBN;
+  __shared__ __align__(16) uint16_t As[2][GBM * GBK];
+  __shared__ __align__(16) uint16_t Bs[2][GBN * GBK];
+  // workgroup b runs on XCD b % 8: each XCD takes a contiguous range of tiles (n fastest), so the
+  // operand that a row of tiles shares comes into one L2 instead of eight
+  const unsigned tiles = gridDim.x * gridDim.y, id = blockIdx.x + gridDim.x * blockIdx.y;
+  const unsigned tile = (id & 7) * (tiles >> 3) + min(id & 7, tiles & 7) + (id >> 3);
+  const int m0 = (int)(tile / gridDim.x) * GBM, n0 = (int)(tile % gridDim.x) * GBN;
   const int kb = blockIdx.z * kchunk;
   const int ke = min(K, kb + kchunk);
   float* cz = c + (long long)blockIdx.z * M * N;
@@ -99,21 +168,46 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(int M, int N, int K, int
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int kq = (lane >> 4) * 8;
-  for (int k0 = kb; k0 < ke; k0 += GBK) {
-    load_tile(a, sam, sak, M, m0, k0, ke, As, t);
-    load_tile(b, sbn, sbk, N, n0, k0, ke, Bs, t);  // B viewed as (n, k)
+  const int steps = (ke - kb + GBK - 1) / GBK;
+  GemmFrag fa[2], fb[2];
+  fa[0] = gemm_load<AK, WIDE>(a, sam, sak, M, m0, kb, ke, t);
+  fb[0] = gemm_load<BK, WIDE>(b, sbn, sbk, N, n0, kb, ke, t);  // B viewed as (n, k)
+  fa[1] = gemm_load<AK, WIDE>(a, sam, sak, M, m0, kb + GBK, ke, t);
+  fb[1] = gemm_load<BK, WIDE>(b, sbn, sbk, N, n0, kb + GBK, ke, t);
+  auto step = [&](int s, GemmFrag& ra, GemmFrag& rb) {
+    // buffer s & 1 was last read in step s - 2; the barrier of step s - 1 lies in between
+    gemm_store<AK>(ra, As[s & 1], t);
+    gemm_store<BK>(rb, Bs[s & 1], t);
+    // past the last step the loads are masked: issued all the same, so that the compiler knows
+    // how many are in flight and waits for the older step's only
+    ra = gemm_load<AK, WIDE>(a, sam, sak, M, m0, kb + (s + 2) * GBK, ke, t);
+    rb = gemm_load<BK, WIDE>(b, sbn, sbk, N, n0, kb + (s + 2) * GBK, ke, t);
     __syncthreads();
-    bf16x8 av[2], bv[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) av[i] = *reinterpret_cast<const bf16x8*>(&As[(wm * 32 + i * 16 + (lane & 15)) * GLD + kq]);
+    for (int h = 0; h < 2; ++h) {
+      bf16x8 av[2], bv[2];
+      const int chunk = (lane >> 4) + 4 * h;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) bv[j] = *reinterpret_cast<const bf16x8*>(&Bs[(wn * 32 + j * 16 + (lane & 15)) * GLD + kq]);
+      for (int i = 0; i < 2; ++i) {
+        const int r = wm * 32 + i * 16 + (lane & 15);
+        av[i] = *reinterpret_cast<const bf16x8*>(&As[s & 1][r * GBK + gswz(r, chunk) * 8]);
+      }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+      for (int j = 0; j < 2; ++j) {
+        const int r = wn * 32 + j * 16 + (lane & 15);
+        bv[j] = *reinterpret_cast<const bf16x8*>(&Bs[s & 1][r * GBK + gswz(r, chunk) * 8]);
+      }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
+    }
+  };
+  for (int s = 0;;) {
+    step(s, fa[0], fb[0]);
+    if (++s >= steps) break;
+    step(s, fa[1], fb[1]);
+    if (++s >= steps) break;
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -134,19 +228,37 @@ int gemm_bf16(int M, int N, int K, const uint16_t* a, long long sam, long long s
   splits = std::max(1, splits);
   const int kchunk = (int)ceil_div(ceil_div(K, splits), GBK) * GBK;
   const int z = (int)ceil_div(K, kchunk);
-  hipLaunchKernelGGL(gemm_bf16_kernel, dim3((N + GBN - 1) / GBN, (M + GBM - 1) / GBM, z), dim3(256), 0, s, M, N, K,
-                     kchunk, a, sam, sak, b, sbk, sbn, c);
+  const dim3 grid((N + GBN - 1) / GBN, (M + GBM - 1) / GBM, z);
+  const bool wide = gemm_wide(a, M, K, sam, sak) && gemm_wide(b, N, K, sbn, sbk);
+#define PP_GEMM(AK, BK)                                                                                              \
+  if (wide)                                                                                                          \
+    hipLaunchKernelGGL((gemm_bf16_kernel<AK, BK, true>), grid, dim3(256), 0, s, M, N, K, kchunk, a, sam, sak, b, sbk, \
+                       sbn, c);                                                                                      \
+  else                                                                                                               \
+    hipLaunchKernelGGL((gemm_bf16_kernel<AK, BK, false>), grid, dim3(256), 0, s, M, N, K, kchunk, a, sam, sak, b,     \
+                       sbk, sbn, c)
+  if (sak == 1 && sbk == 1) {
+    PP_GEMM(true, true);
+  } else if (sak == 1) {
+    PP_GEMM(true, false);
+  } else if (sbk == 1) {
+    PP_GEMM(false, true);
+  } else {
+    PP_GEMM(false, false);
+  }
+#undef PP_GEMM
   PP_HIP(hipGetLastError());
   return z;
 }
 
-// Split-K factor: enough workgroups for the chip (about 256), at most 32 splits and at
-// least 128 of K per split.  Skinny products (the inference of a few dozen channel rows)
+// Split-K factor: enough workgroups for the chip (about 512), at most 32 splits and at
+// least 128 of K per split (256 x 512 x 7200: 8 splits 12 us, 15 splits 10).  Skinny products (the
+// inference of a few dozen channel rows)
 // split most.
 constexpr int kOutSplitsMax = 4;  // split-K of the output layer (its partials are rows x in)
 static int pick_splits(int M, int N, int K) {
   const long long tiles = ceil_div(M, GBM) * ceil_div(N, GBN);
-  int sp = (int)std::max(1LL, 256 / std::max(1LL, tiles));
+  int sp = (int)std::max(1LL, 512 / std::max(1LL, tiles));
   sp = std::min(sp, 32);
   sp = std::min(sp, std::max(1, K / 128));
   return sp;
@@ -463,18 +575,6 @@ union BfPack {  // eight BF16 values as one MFMA operand
 };
 
 constexpr int INP = 128;  // FP64 partial sums of squares behind the inference input's norm
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-
-// 16 bytes at byte offset off of the buffer behind r (range-checked: zeros past its end, so a
-// masked-out lane passes kOff16 and its load needs no branch)
-constexpr int kOff16 = 0x7ffffff0;  // beyond every buffer read this way (all under 2 GiB)
-__device__ __forceinline__ u32x4 ld16(__amdgpu_buffer_rsrc_t r, int off) {
-  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-}
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, long long bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
-}
-
 // n2p[b] = sum of squares (FP64) over the b-th of INP equal contiguous ranges of the nf floats
 // of v (nf < 2^29).  Each pass of a thread issues its four 16-byte loads before summing them in
 // order; the range ends (nf, or v not 16-byte aligned) are summed value by value.

@@ -68,3 +68,31 @@ def test_gradients_at_tile_edges(torch, dims):
         assert _rel(g[name], g_ref[name]) < 2e-3, name
     for c in set(range(nchan)) - set(chan.tolist()):
         assert np.all(g["emb"][c] == 0)
+
+
+def _bf16_bits(a):
+    return (mlp.bf16(a).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+
+
+# around the 64 x 64 x 64 tile: below it, exact, one over, K steps 1 to 5 (two are loaded ahead),
+# extents that forbid 16-byte loads
+@pytest.mark.parametrize("a_k", [True, False])
+@pytest.mark.parametrize("b_k", [True, False])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (64, 64, 64), (65, 63, 129), (128, 72, 192), (40, 200, 264), (66, 130, 320)],
+                         ids=lambda d: "x".join(map(str, d)))
+def test_gemm_at_tile_edges(torch, dims, a_k, b_k):
+    from pyprop_amd import _native as N, device as D
+    M, N_, K = dims
+    rng = np.random.default_rng(M * K)
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N_)).astype(np.float32)
+    sam, sak = (K, 1) if a_k else (1, M)
+    sbk, sbn = (1, K) if b_k else (N_, 1)
+    da = torch.from_numpy(_bf16_bits(A if a_k else A.T.copy()).view(np.int16).copy()).to("cuda")
+    db = torch.from_numpy(_bf16_bits(B.T.copy() if b_k else B).view(np.int16).copy()).to("cuda")
+    dc = torch.full((M + 1, N_), 7.0, dtype=torch.float32, device="cuda")
+    N.check(N.load().pp_gemm_bf16(M, N_, K, D.ptr(da), sam, sak, D.ptr(db), sbk, sbn, D.ptr(dc), D.stream_handle()))
+    got = dc.cpu().numpy().astype(np.float64)
+    assert np.all(got[M] == 7.0)  # nothing past the result
+    # exact products of BF16 values, K FP32 additions
+    bound = K * 2.0 ** -24 * (np.abs(mlp.bf16(A)) @ np.abs(mlp.bf16(B)))
+    assert np.all(np.abs(got[:M] - mlp.bf16(A) @ mlp.bf16(B)) <= bound + 1e-30)
