@@ -96,3 +96,25 @@ def test_gemm_at_tile_edges(torch, dims, a_k, b_k):
     # exact products of BF16 values, K FP32 additions
     bound = K * 2.0 ** -24 * (np.abs(mlp.bf16(A)) @ np.abs(mlp.bf16(B)))
     assert np.all(np.abs(got[:M] - mlp.bf16(A) @ mlp.bf16(B)) <= bound + 1e-30)
+
+
+# parameter counts with and without a remainder of two past the 16-byte groups, hidden widths whose
+# matrices start at every offset the layout allows
+@pytest.mark.parametrize("dims", [(1, 1, 8, 3), (5, 3, 72, 15), (3, 4, 64, 40)], ids=lambda d: "x".join(map(str, d)))
+def test_adam_step_and_bf16_copies(torch, dims):
+    nchan, n, hidden, rows = dims
+    net, flat, x, t, chan = _case(nchan, n, hidden, rows, 4)
+    inp = 2 * n * n
+    dev = [torch.from_numpy(a).to("cuda") for a in (x, chan, t)]
+    ref = flat.astype(np.float64)
+    m, v = np.zeros_like(ref), np.zeros_like(ref)
+    for step in (1, 2):
+        net.train_step(*dev, 1e-2)
+        mlp.adam_step(ref, net.get_grads().astype(np.float64), m, v, step, 1e-2)
+        # a step of lr 1e-2 in FP32: a few ulp of the update and of the parameter
+        assert np.max(np.abs(net.get_params() - ref)) < 4 * 2.0 ** -24 * (1.0 + np.max(np.abs(ref)))
+        ref = net.get_params().astype(np.float64)
+    # the next forward pass multiplies with the updated weights, rounded to BF16
+    y = net.forward(dev[0], dev[1]).cpu().numpy().astype(np.float64)
+    y_ref, _ = mlp.forward(mlp.unpack(ref, inp, hidden, nchan), x, chan)
+    assert _rel(y, y_ref) < 1e-4  # one BF16 boundary case in thousands of activations
