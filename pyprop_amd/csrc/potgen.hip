@@ -23,6 +23,17 @@
 // [q][v] tile read 16 bytes at a time and chunked weight loads were all slower (fewer
 // resident waves).
 //
+// Two radial ranks, few terms: the potential is linear in its terms, so with many more angular
+// pairs than terms the grid function of each term is projected once, R[t] (P1 x P2, in the
+// caller's work buffer), and every pair's block is written as sum_t C[t][a] R[t]
+// (expand_terms_kernel, tensorpotential.hip).  Projecting each pair's own grid function spends
+// 49 FMAs per written element twice over and was bound by LDS reads: helium R12 (394 pairs, 11
+// terms, 3.63 GB written) 0.80 + 3.06 ms, this way
+// 0.04 + 0.07 + 0.70 ms.  It needs room for the T intermediate
+// and T projected functions in the work buffer that holds one intermediate per pair:
+// T (Q1 + P1) <= P0 Q1; below that line (T > P0 / 3 at the usual P1 = 2 Q1) there is little to
+// gain, and the pairs are projected one by one.
+//
 // Grid functions on the device:
 //  * multipole: F[a][q1][q2] = sum_l C[l][a] r<^l / r>^(l+1), the 1/r12 expansion that
 //    CustomPotentialEvaluationR12 evaluates on the (q1, q2) grid
@@ -123,6 +134,32 @@ struct SeparableSource {
       v = fma(C[(long long)t * P0 + a] * g1, f2[(long long)t * n2 + q2], v);
     }
     return v;
+  }
+};
+
+// row r = t * n1 + q1 of term t alone, without its coefficients: r<^lam_t / r>^(lam_t + 1)
+struct MultipoleTermSource {
+  int n1;
+  const int* lams;
+  const double* r1;
+  const double* r2;
+  __device__ double operator()(long long r, int q2) const {
+    const int t = (int)(r / n1), q1 = (int)(r - (long long)t * n1);
+    const double x1 = r1[q1], x2 = r2[q2];
+    const double rlo = fmin(x1, x2), rhi = fmax(x1, x2);
+    const double ratio = rlo / rhi;
+    double pw = 1.0;
+    for (int l = 0; l < lams[t]; ++l) pw *= ratio;
+    return pw / rhi;
+  }
+};
+// row r = t * n1 + q1 of f1[t][q1] f2[t][q2]
+struct SeparableTermSource {
+  int n1, n2;
+  const double* f1;
+  const double* f2;
+  __device__ double operator()(long long r, int q2) const {
+    return f1[r] * f2[(r / n1) * n2 + q2];
   }
 };
 
@@ -321,6 +358,21 @@ static void launch_cols(const BsProjection& P, long long pre, long long post, co
   PP_HIP(hipGetLastError());
 }
 
+// Whether the terms are projected and then combined (the work buffer holds P0 Q1 P2 values)
+static bool project_terms(const BsProjection& A, long long P0, long long terms) {
+  return terms * ((long long)A.Q + A.P) <= P0 * A.Q;
+}
+
+// dst[a] (+)= sum_t coeffs[t][a] R[t] with R[t] the projection of row source `term` (T Q1 rows)
+template <typename SRC>
+static void represent_terms(const BsProjection& A, const BsProjection& B, long long P0, int terms, SRC term,
+                            const double* coeffs, double* work, double2* dst, int accumulate, hipStream_t s) {
+  double* radial = work + (long long)terms * A.Q * B.P;
+  launch_rows(B, (long long)terms * A.Q, term, work, 0, s);
+  launch_cols(A, (long long)terms, (long long)B.P, work, radial, 0, s);
+  expand_terms(terms, P0, (long long)A.P * B.P, coeffs, radial, dst, accumulate, s);
+}
+
 }  // namespace pp
 
 extern "C" int pp_bspline_represent(const pp_bspline_projection* proj, int64_t pre, int64_t post, const double* src,
@@ -356,6 +408,11 @@ extern "C" int pp_potential_represent_multipole(const pp_bspline_projection* pro
     const BsProjection& A = proj1->p;
     const BsProjection& B = proj2->p;
     const hipStream_t s = (hipStream_t)stream;
+    if (project_terms(A, pair_count, nlam)) {
+      represent_terms(A, B, pair_count, nlam, MultipoleTermSource{A.Q, lams, r1, r2}, coeffs, work,
+                      reinterpret_cast<double2*>(dst), accumulate, s);
+      return;
+    }
     const MultipoleSource in{(long long)pair_count, nlam, A.Q, lams, coeffs, r1, r2};
     launch_rows(B, (long long)pair_count * A.Q, in, work, 0, s);
     launch_cols(A, (long long)pair_count, (long long)B.P, work, reinterpret_cast<double2*>(dst), accumulate, s);
@@ -379,6 +436,11 @@ extern "C" int pp_potential_represent_separable(const pp_bspline_projection* pro
     }
     PP_REQUIRE(f2 && work, "null argument");
     const BsProjection& B = proj2->p;
+    if (project_terms(A, pair_count, terms)) {
+      represent_terms(A, B, pair_count, terms, SeparableTermSource{A.Q, B.Q, f1, f2}, coeffs, work,
+                      reinterpret_cast<double2*>(dst), accumulate, s);
+      return;
+    }
     const SeparableSource in{(long long)pair_count, terms, A.Q, B.Q, coeffs, f1, f2};
     launch_rows(B, (long long)pair_count * A.Q, in, work, 0, s);
     launch_cols(A, (long long)pair_count, (long long)B.P, work, reinterpret_cast<double2*>(dst), accumulate, s);

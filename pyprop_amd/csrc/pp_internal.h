@@ -70,6 +70,11 @@ void tp_run_f32(const TPPlanDevice& plan, const std::vector<const TPTerm*>& term
                 float2 alpha, bool accumulate, hipStream_t s);
 void tp_ensure_f32(const TPTerm& t, hipStream_t s);
 
+// out[a][r] (+)= sum_t coeffs[t][a] radial[t][r] for a < p0, r < rc (the real part; a first write
+// sets the imaginary part to zero)
+void expand_terms(int terms, long long p0, long long rc, const double* coeffs, const double* radial, double2* out,
+                  int accumulate, hipStream_t s);
+
 // BLAS-1 helpers (blas.hip)
 struct Reducer {
   // scratch for two-stage deterministic reductions
