@@ -61,8 +61,7 @@ extern "C" int pp_repr_inner_product(const pp_repr* repr, const pp_cplx* a, cons
     hipStream_t s = (hipStream_t)stream;
     const long long n = repr->r.size();
     double2* w = reinterpret_cast<double2*>(work);
-    vec_copy(n, reinterpret_cast<const double2*>(b), w, s);
-    repr->r.overlap(PP_OVERLAP_MULTIPLY, false, w, s);
+    repr->r.overlap_into(PP_OVERLAP_MULTIPLY, false, reinterpret_cast<const double2*>(b), w, s);
     Reducer red;
     red.ensure(reduction_blocks(n), 2);
     vec_dot(n, reinterpret_cast<const double2*>(a), w, red.result.ptr, red, s);

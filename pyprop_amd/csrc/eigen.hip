@@ -401,8 +401,7 @@ struct ShiftInvert {
       double2* out = reinterpret_cast<double2*>(out_);
       hipStream_t s = (hipStream_t)s_;
       const long long n = si->ham->n;
-      vec_copy(n, in, si->tmp.ptr, s);
-      si->ham->repr->overlap(PP_OVERLAP_MULTIPLY, false, si->tmp.ptr, s);
+      si->ham->repr->overlap_into(PP_OVERLAP_MULTIPLY, false, in, si->tmp.ptr, s);
       vec_combine(n, make_double2(-si->shift, 0), si->tmp.ptr, make_double2(0, 0), nullptr, si->tmp.ptr, s);
       if (si->fham) fham_apply64(*si->fham, si->scalings.data(), in, out, si->tmp.ptr, make_double2(1.0, 0), s);
       else si->ham->apply(si->scalings.data(), in, out, si->tmp.ptr, make_double2(1.0, 0), s);
@@ -416,8 +415,7 @@ struct ShiftInvert {
   // InverseIterations (GMRESShiftInvertSolver.py:100-126)
   void solve(const double2* b, double2* x, hipStream_t s) {
     const long long n = ham->n;
-    vec_copy(n, b, rhs.ptr, s);
-    ham->repr->overlap(PP_OVERLAP_MULTIPLY, false, rhs.ptr, s);
+    ham->repr->overlap_into(PP_OVERLAP_MULTIPLY, false, b, rhs.ptr, s);
     if (pc) precond_solve(*pc, rhs.ptr, s);
     gmres.solve(&ShiftInvert::op_cb, this, rhs.ptr, x, s);
     ++solves;

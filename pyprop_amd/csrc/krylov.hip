@@ -33,9 +33,13 @@ using cd = std::complex<double>;
 // ----------------------------------------------------------------------------------
 // representation
 // ----------------------------------------------------------------------------------
-void Repr::overlap(int op, bool conj, double2* psi, hipStream_t s, double2* work) const {
-  for (int r = 0; r < ndim; ++r)
-    if (ov[r]) overlap_apply(*ov[r], op, conj, ndim, extents.data(), r, psi, s, work);
+void Repr::overlap_into(int op, bool conj, const double2* src, double2* dst, hipStream_t s, double2* work) const {
+  for (int r = 0; r < ndim; ++r) {
+    if (!ov[r]) continue;
+    overlap_apply(*ov[r], op, conj, ndim, extents.data(), r, src, dst, s, work);
+    src = dst;
+  }
+  if (src != dst) vec_copy(size(), src, dst, s);
 }
 
 // ----------------------------------------------------------------------------------
@@ -69,8 +73,7 @@ void Hamiltonian::apply_f32(const double* scalings, const float2* src, float2* d
 
 void Hamiltonian::multiply_balanced(const double* scalings, const double2* src, double2* dst, hipStream_t s) {
   ensure_work();
-  vec_copy(n, src, work.ptr, s);
-  repr->overlap(PP_OVERLAP_SQRT_SOLVE, false, work.ptr, s);
+  repr->overlap_into(PP_OVERLAP_SQRT_SOLVE, false, src, work.ptr, s);
   apply(scalings, work.ptr, dst, nullptr, make_double2(1.0, 0.0), s);
   repr->overlap(PP_OVERLAP_SQRT_SOLVE, true, dst, s);
 }
@@ -492,8 +495,7 @@ int Cayley::operator_cb(void* ctx, const pp_cplx* in_, pp_cplx* out_, pp_stream 
     double2* out = reinterpret_cast<double2*>(out_);
     hipStream_t s = (hipStream_t)s_;
     // SolverCallback: MultiplySpH(+i dt/2) then left preconditioner (CayleyPropagator.py:145-150)
-    vec_copy(c->n, in, c->tmp_s.ptr, s);
-    c->ham->repr->overlap(PP_OVERLAP_MULTIPLY, false, c->tmp_s.ptr, s);
+    c->ham->repr->overlap_into(PP_OVERLAP_MULTIPLY, false, in, c->tmp_s.ptr, s);
     if (c->fham) fham_apply64(*c->fham, c->scalings.data(), in, out, c->tmp_s.ptr, make_double2(0.0, 0.5 * c->dt), s);
     else c->ham->apply(c->scalings.data(), in, out, c->tmp_s.ptr, make_double2(0.0, 0.5 * c->dt), s);
     if (c->pc) precond_solve(*c->pc, out, s);
@@ -509,8 +511,7 @@ void Cayley::step(double2* psi, double dt_, const double* sc, hipStream_t s) {
   dt = dt_;
   scalings.assign(sc, sc + ham->terms.size());
   // TempPsi = (S - i dt/2 H) psi   (AdvanceStep, CayleyPropagator.py:81-85)
-  vec_copy(n, psi, tmp_s.ptr, s);
-  ham->repr->overlap(PP_OVERLAP_MULTIPLY, false, tmp_s.ptr, s);
+  ham->repr->overlap_into(PP_OVERLAP_MULTIPLY, false, psi, tmp_s.ptr, s);
   if (fham) fham_apply64(*fham, scalings.data(), psi, rhs.ptr, tmp_s.ptr, make_double2(0.0, -0.5 * dt), s);
   else ham->apply(scalings.data(), psi, rhs.ptr, tmp_s.ptr, make_double2(0.0, -0.5 * dt), s);
   if (pc) precond_solve(*pc, rhs.ptr, s);

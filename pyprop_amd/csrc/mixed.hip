@@ -1876,8 +1876,7 @@ void MixedCayley::step(double2* psi, double dt, const double* sc, hipStream_t s)
         return;
       }
     } else {
-      vec_copy(n, psi, work.t64.ptr, cs);
-      R.overlap(PP_OVERLAP_MULTIPLY, false, work.t64.ptr, cs);
+      R.overlap_into(PP_OVERLAP_MULTIPLY, false, psi, work.t64.ptr, cs);
       if (fham) fham->apply64(scal.data(), psi, work.h64.ptr, nullptr, make_double2(1.0, 0.0), cs,
                               make_double2(0.0, 0.0), scd);
       else H.apply(scal.data(), psi, work.h64.ptr, nullptr, make_double2(1.0, 0.0), cs);
@@ -1949,8 +1948,7 @@ void MixedCayley::step(double2* psi, double dt, const double* sc, hipStream_t s)
       fham->apply64(scal.data(), work.x64.ptr, work.r64.ptr, nullptr, make_double2(0.0, a), cs,
                     make_double2(1.0, 0.0), scd);
     } else {
-      vec_copy(n, work.x64.ptr, work.t64.ptr, cs);
-      R.overlap(PP_OVERLAP_MULTIPLY, false, work.t64.ptr, cs);
+      R.overlap_into(PP_OVERLAP_MULTIPLY, false, work.x64.ptr, work.t64.ptr, cs);
       if (fham) fham->apply64(scal.data(), work.x64.ptr, work.r64.ptr, work.t64.ptr, make_double2(0.0, a), cs,
                               make_double2(0.0, 0.0), scd);
       else H.apply(scal.data(), work.x64.ptr, work.r64.ptr, work.t64.ptr, make_double2(0.0, a), cs);

@@ -4,10 +4,16 @@
 //   solve     x <- U^-1 (U^-H x)    (ztbsv 'U','C' then 'N', :130-135)
 //   sqrt      x <- U x | U^H x, x <- U^-1 x | U^-H x (:137-149)
 // applied to every 1-D fibre of one rank of a C-ordered tensor (MapToRank3 loops,
-// :155-229).  One thread owns one fibre; consecutive threads own consecutive
-// trailing indices, so loads are coalesced whenever the rank is not the last one.
+// :155-229).
+//
+// Up to kTileRows rows a workgroup holds a tile of whole fibres in LDS: the multiplies are banded
+// sums out of LDS and S^-1 x is a product with the dense inverse, which the host forms in extended
+// precision (overlap_tile_kernel); U^-1 x and U^-H x are substitutions by one lane per fibre with
+// the rows and coefficients staged (overlap_chain_kernel).  Beyond, one thread owns one fibre
+// (substitution) or one element (multiply).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -92,8 +98,8 @@ __global__ void overlap_fibre_kernel(const double* __restrict__ u, int n, int sd
   else { if (CONJ) solve_uh(); else solve_u(); }
 }
 
-// Same operations with the band width fixed at compile time: each thread keeps a sliding
-// window of SD+1 fibre values in registers, so every element of the fibre is loaded and
+// The solves with the band width fixed at compile time: each thread keeps a sliding
+// window of the last SD unknowns in registers, so every element of the fibre is loaded and
 // stored exactly once per pass and the recurrences run out of registers.  The band
 // coefficients of row/column i are uniform across the wave (scalar loads).
 template <int OP, bool CONJ, int SD>
@@ -105,49 +111,6 @@ __global__ __launch_bounds__(128) void overlap_window_kernel(const double* __res
   double2* x = data + p * n * post + q;
   const long long st = post;
   auto U = [&](int i, int j) { return u[j * (SD + 1) + SD + i - j]; };
-  auto ld = [&](int i) { return (i >= 0 && i < n) ? x[i * st] : make_double2(0, 0); };
-  // x <- U x, ascending: x_i = sum_{d=0..SD} U(i, i+d) x_{i+d} (old values)
-  auto mul_u = [&]() {
-    double2 w[SD + 1];
-#pragma unroll
-    for (int d = 0; d <= SD; ++d) w[d] = ld(d);
-    for (int i = 0; i < n; ++i) {
-      double2 acc = make_double2(0, 0);
-#pragma unroll
-      for (int d = 0; d <= SD; ++d) {
-        if (i + d < n) {
-          const double a = U(i, i + d);
-          acc.x = fma(a, w[d].x, acc.x);
-          acc.y = fma(a, w[d].y, acc.y);
-        }
-      }
-      x[i * st] = acc;
-#pragma unroll
-      for (int d = 0; d < SD; ++d) w[d] = w[d + 1];
-      w[SD] = ld(i + SD + 1);
-    }
-  };
-  // x <- U^H x, descending: x_i = sum_{d=0..SD} U(i-d, i) x_{i-d} (old values)
-  auto mul_uh = [&]() {
-    double2 w[SD + 1];
-#pragma unroll
-    for (int d = 0; d <= SD; ++d) w[d] = ld(n - 1 - d);
-    for (int i = n - 1; i >= 0; --i) {
-      double2 acc = make_double2(0, 0);
-#pragma unroll
-      for (int d = 0; d <= SD; ++d) {
-        if (i - d >= 0) {
-          const double a = U(i - d, i);
-          acc.x = fma(a, w[d].x, acc.x);
-          acc.y = fma(a, w[d].y, acc.y);
-        }
-      }
-      x[i * st] = acc;
-#pragma unroll
-      for (int d = 0; d < SD; ++d) w[d] = w[d + 1];
-      w[SD] = ld(i - SD - 1);
-    }
-  };
   // x <- U^-1 x, descending; window holds the SD most recently solved values x_{i+1..i+SD}
   auto solve_u = [&]() {
     double2 w[SD + 1];
@@ -194,9 +157,7 @@ __global__ __launch_bounds__(128) void overlap_window_kernel(const double* __res
       w[0] = acc;
     }
   };
-  if (OP == PP_OVERLAP_MULTIPLY) { mul_u(); mul_uh(); }
-  else if (OP == PP_OVERLAP_SOLVE) { solve_uh(); solve_u(); }
-  else if (OP == PP_OVERLAP_SQRT_MULTIPLY) { if (CONJ) mul_uh(); else mul_u(); }
+  if (OP == PP_OVERLAP_SOLVE) { solve_uh(); solve_u(); }
   else { if (CONJ) solve_uh(); else solve_u(); }
 }
 
@@ -227,17 +188,303 @@ __global__ __launch_bounds__(256) void overlap_elem_kernel(const double* __restr
   y[idx] = acc;
 }
 
+constexpr int kTileRows = 512;
+
+// A tile of FT fibres: where it starts, how many fibres it has, and the strides of a row and of a
+// fibre (consecutive fibres are neighbours in memory when the rank is not the last one).
+struct FibreTile {
+  long long base, row, fibre;
+  int cnt;
+};
+template <int FT>
+__device__ inline FibreTile fibre_tile(int n, long long pre, long long post) {
+  if (post > 1) {
+    const long long tiles = (post + FT - 1) / FT, p = blockIdx.x / tiles, q0 = (blockIdx.x - p * tiles) * FT;
+    return {p * n * post + q0, post, 1, (int)min((long long)FT, post - q0)};
+  }
+  const long long p0 = blockIdx.x * (long long)FT;
+  return {p0 * n, 1, n, (int)min((long long)FT, pre - p0)};
+}
+// element e of the tile in memory order: consecutive threads on consecutive addresses
+template <int FT>
+__device__ inline void tile_element(const FibreTile& t, int n, int e, int& i, int& f) {
+  if (t.row > 1) {
+    i = e / FT;
+    f = e % FT;
+  } else {
+    f = e / n;
+    i = e - f * n;
+  }
+}
+template <int FT>
+__device__ inline void load_tile(const FibreTile& t, int n, const double2* src, double2* X) {
+  for (int e = threadIdx.x; e < n * FT; e += blockDim.x) {
+    int i, f;
+    tile_element<FT>(t, n, e, i, f);
+    X[i * FT + f] = f < t.cnt ? src[t.base + i * t.row + f * t.fibre] : make_double2(0, 0);
+  }
+}
+static long long tile_count(long long pre, long long post, int ft) {
+  return post > 1 ? pre * ((post + ft - 1) / ft) : (pre + ft - 1) / ft;
+}
+
+// Without Sinv: x <- U x, U^H x or U^H (U x), in the order of the sums above.  With it: x <- S^-1 x,
+// S^-1 as rows [j][i] of which lanes i read consecutive values: wave (g, k) sums rows
+// 64 g .. 64 g + 63 over the k-th part of j for all FT fibres, and the parts are added in order.
+// dst may be src: a workgroup has read its tile before it writes it.  Two substitutions are a chain
+// of 2 n dependent rows with one lane per fibre, 50.5 us per rank at 42 x 60 x 60; the product has
+// none, 10.9 us.  The two banded passes of U^H U in one launch: 2 x 5.0 us -> 5.6.
+template <int FT>
+__global__ __launch_bounds__(1024) void overlap_tile_kernel(const double* __restrict__ u,
+                                                            const double* __restrict__ Sinv, int mul_first,
+                                                            int mul_second, int n, int sd, int parts, long long pre,
+                                                            long long post, const double2* src, double2* dst) {
+  extern __shared__ double2 tile[];
+  double2* X = tile;           // [n][FT]
+  double2* Y = tile + n * FT;  // [parts][n][FT]
+  const FibreTile t = fibre_tile<FT>(n, pre, post);
+  load_tile<FT>(t, n, src, X);
+  if (!Sinv) {
+    double* C = reinterpret_cast<double*>(tile + 2 * n * FT);
+    for (int e = threadIdx.x; e < n * (sd + 1); e += blockDim.x) C[e] = u[e];
+    __syncthreads();
+    auto band = [&](const double2* in, int mode, int i, int f) {
+      double2 acc = make_double2(0, 0);
+      const int step = mode == 0 ? 1 : -1;
+#pragma unroll 4
+      for (int d = 0; d <= sd; ++d) {
+        const int j = i + step * d;
+        const bool in_range = j >= 0 && j < n;
+        const double c = C[(mode == 0 && in_range ? j : i) * (sd + 1) + sd - d];
+        const double2 x = in[(in_range ? j : i) * FT + f];
+        acc.x = in_range ? fma(c, x.x, acc.x) : acc.x;
+        acc.y = in_range ? fma(c, x.y, acc.y) : acc.y;
+      }
+      return acc;
+    };
+    const double2* last = X;
+    if (mul_second >= 0) {
+      for (int e = threadIdx.x; e < n * FT; e += blockDim.x) Y[e] = band(X, mul_first, e / FT, e % FT);
+      __syncthreads();
+      last = Y;
+    }
+    const int mode = mul_second >= 0 ? mul_second : mul_first;
+    for (int e = threadIdx.x; e < n * FT; e += blockDim.x) {
+      int i, f;
+      tile_element<FT>(t, n, e, i, f);
+      if (f < t.cnt) dst[t.base + i * t.row + f * t.fibre] = band(last, mode, i, f);
+    }
+    return;
+  }
+  __syncthreads();
+  const int groups = (n + 63) / 64, wave = threadIdx.x >> 6, g = wave % groups, k = wave / groups;
+  const int i = 64 * g + (threadIdx.x & 63);
+  const int j0 = n * k / parts, j1 = n * (k + 1) / parts;
+  if (i < n) {
+    double2 acc[FT];
+#pragma unroll
+    for (int f = 0; f < FT; ++f) acc[f] = make_double2(0, 0);
+#pragma unroll 8
+    for (int j = j0; j < j1; ++j) {
+      const double m = Sinv[(long long)j * n + i];
+#pragma unroll
+      for (int f = 0; f < FT; ++f) {
+        const double2 x = X[j * FT + f];
+        acc[f].x = fma(m, x.x, acc[f].x);
+        acc[f].y = fma(m, x.y, acc[f].y);
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < FT; ++f) Y[(k * n + i) * FT + f] = acc[f];
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n * FT; e += blockDim.x) {
+    int r, f;
+    tile_element<FT>(t, n, e, r, f);
+    if (f >= t.cnt) continue;
+    double2 s = Y[r * FT + f];
+    for (int p = 1; p < parts; ++p) {
+      s.x += Y[(p * n + r) * FT + f].x;
+      s.y += Y[(p * n + r) * FT + f].y;
+    }
+    dst[t.base + r * t.row + f * t.fibre] = s;
+  }
+}
+
+static void overlap_tile(const OverlapFactor& ov, int op, bool conj, long long pre, long long post, const double2* src,
+                         double2* dst, hipStream_t s) {
+  const int n = ov.n, groups = (n + 63) / 64;
+  const long long fibres = pre * post;
+  const bool solve = op == PP_OVERLAP_SOLVE;
+  const int first = op == PP_OVERLAP_MULTIPLY ? 0 : conj ? 1 : 0, second = op == PP_OVERLAP_MULTIPLY ? 1 : -1;
+  // few fibres: one per workgroup, so that as many CUs as there are take part; many: tiles whose
+  // coefficients are read once for FT fibres, as wide as leaves 64 KB of LDS for the partial sums
+  const int ft = fibres <= 512 ? 1 : n <= 64 ? (solve ? 8 : 4) : n <= 160 ? 4 : n <= 320 ? 2 : 1;
+  const int parts = solve ? std::max(1, std::min(ft >= 4 ? 4 : 8, 16 / groups)) : 1;
+  const int threads = solve ? 64 * groups * parts : 256;
+  const size_t lds = (size_t)n * ft * (1 + parts) * sizeof(double2) + (solve ? 0 : (size_t)n * (ov.sd + 1) * sizeof(double));
+  const long long blocks = tile_count(pre, post, ft);
+  PP_REQUIRE(blocks <= 0x7fffffffLL, "too many fibres");
+#define PP_TILE(F)                                                                                             \
+  case F:                                                                                                      \
+    hipLaunchKernelGGL(overlap_tile_kernel<F>, dim3((unsigned)blocks), dim3(threads), lds, s, ov.u.ptr,        \
+                       solve ? ov.s_inv.ptr : nullptr, first, second, n, ov.sd, parts, pre, post, src, dst);   \
+    break;
+  switch (ft) {
+    PP_TILE(1) PP_TILE(2) PP_TILE(4) PP_TILE(8)
+  }
+#undef PP_TILE
+  PP_HIP(hipGetLastError());
+}
+
+// x / c for r = 1 / c rounded: two residual corrections of x r give the rounded quotient (P. Markstein,
+// IBM J. Res. Dev. 34 (1990) 111), the bits of the division (0 for x = -0), in five dependent
+// operations instead of its ten.  Where a residual could underflow or a value is not finite (r NaN:
+// a divisor outside 2^+-100) the division itself, behind a branch of the whole wave: the compiler
+// would otherwise compute both.
+__device__ inline double divide_by(double x, double c, double r) {
+  double q = x * r;
+  const bool plain = (fabs(q) > 1e-250 && fabs(q) < 1e250) || x == 0.0;
+  q = fma(fma(-q, c, x), r, q);
+  q = fma(fma(-q, c, x), r, q);
+  if (__ballot(!plain)) q = plain ? q : x / c;
+  return q;
+}
+
+// x <- U^-1 x (LOWER false, descending rows) or U^-H x (ascending) with the arithmetic of
+// overlap_window_kernel, term by term: a Krylov exponential amplifies the rounding of these solves
+// from step to step, so another order of the same sums would move its results.  What is left is the
+// chain itself, SD dependent FMAs and a division per row.  The tile and the coefficients (zeros
+// outside the matrix, then the diagonal and its reciprocal) sit in LDS with the rows in the order
+// they are solved, padded to a multiple of SD by rows that are never read back; U is real, so the
+// real and imaginary parts are solved by lanes of their own in the first wave.  A lane reads two
+// rows ahead and keeps the last SD unknowns in registers that rotate through an unrolled loop.
+// 8 fibres of 120 rows: 58 (U^-1) and 31 us (U^-H) with every row loaded from memory in turn,
+// 14.4 us here; with the compiler's division and a bounds test per row 26.
+template <int SD, int FT, bool LOWER>
+__global__ __launch_bounds__(256) void overlap_chain_kernel(const double* __restrict__ u, int n, int rows,
+                                                            long long pre, long long post, const double2* src,
+                                                            double2* dst) {
+  constexpr int W = SD + 2, P = 2 * FT;
+  extern __shared__ double2 tile[];
+  double2* X = tile;                                              // [rows + 2][FT]
+  double* C = reinterpret_cast<double*>(tile + (rows + 2) * FT);  // [rows + 2][W]
+  const FibreTile t = fibre_tile<FT>(n, pre, post);
+  for (int e = threadIdx.x; e < n * FT; e += blockDim.x) {
+    int i, f;
+    tile_element<FT>(t, n, e, i, f);
+    X[(LOWER ? i : n - 1 - i) * FT + f] = f < t.cnt ? src[t.base + i * t.row + f * t.fibre] : make_double2(0, 0);
+  }
+  for (int e = n * FT + threadIdx.x; e < (rows + 2) * FT; e += blockDim.x) X[e] = make_double2(0, 0);
+  for (int e = threadIdx.x; e < (rows + 2) * (SD + 1); e += blockDim.x) {
+    const int r = e / (SD + 1), d = e % (SD + 1) + 1, i = LOWER ? r : n - 1 - r;
+    if (d <= SD) {
+      double c = 0.0;
+      if (r < n && LOWER && i - d >= 0) c = u[i * (SD + 1) + SD - d];
+      if (r < n && !LOWER && i + d < n) c = u[(i + d) * (SD + 1) + SD - d];
+      C[r * W + d - 1] = c;
+    } else {
+      const double c = r < n ? u[i * (SD + 1) + SD] : 1.0;
+      C[r * W + SD] = c;
+      C[r * W + SD + 1] = c > 0x1p-100 && c < 0x1p100 ? 1.0 / c : __builtin_nan("");
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < P) {
+    double* x = reinterpret_cast<double*>(X) + threadIdx.x;
+    double w[SD];  // the unknown of row r sits in w[r % SD]
+#pragma unroll
+    for (int d = 0; d < SD; ++d) w[d] = 0.0;
+    double xa = x[0], xb = x[P], ca[W], cb[W];
+#pragma unroll
+    for (int d = 0; d < W; ++d) {
+      ca[d] = C[d];
+      cb[d] = C[W + d];
+    }
+    for (int r0 = 0; r0 < rows; r0 += SD) {
+#pragma unroll
+      for (int q = 0; q < SD; ++q) {
+        const int r = r0 + q;
+        const double xc = x[(r + 2) * P];
+        double cc[W];
+#pragma unroll
+        for (int d = 0; d < W; ++d) cc[d] = C[(r + 2) * W + d];
+#pragma unroll
+        for (int d = 1; d <= SD; ++d) xa = fma(-ca[d - 1], w[(q + SD - d) % SD], xa);
+        w[q] = divide_by(xa, ca[SD], ca[SD + 1]);
+        x[r * P] = w[q];
+        xa = xb;
+        xb = xc;
+#pragma unroll
+        for (int d = 0; d < W; ++d) {
+          ca[d] = cb[d];
+          cb[d] = cc[d];
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n * FT; e += blockDim.x) {
+    int i, f;
+    tile_element<FT>(t, n, e, i, f);
+    if (f < t.cnt) dst[t.base + i * t.row + f * t.fibre] = X[(LOWER ? i : n - 1 - i) * FT + f];
+  }
+}
+
+template <int SD>
+static void overlap_chain(const OverlapFactor& ov, bool lower, long long pre, long long post, const double2* src,
+                          double2* dst, hipStream_t s) {
+  // few fibres: two per workgroup (the chain costs the same for any number; the copies shrink);
+  // many: 16, as long as the tile leaves a CU several workgroups
+  const int n = ov.n, ft = pre * post <= 512 || n > 160 ? 2 : 16;
+  const int rows = (n + SD - 1) / SD * SD;
+  const size_t lds = (size_t)(rows + 2) * (ft * sizeof(double2) + (SD + 2) * sizeof(double));
+  const long long blocks = tile_count(pre, post, ft);
+  PP_REQUIRE(blocks <= 0x7fffffffLL, "too many fibres");
+#define PP_CHAIN(F, L)                                                                                             \
+  hipLaunchKernelGGL((overlap_chain_kernel<SD, F, L>), dim3((unsigned)blocks), dim3(256), lds, s, ov.u.ptr, n, rows, \
+                     pre, post, src, dst)
+  if (ft == 2) {
+    if (lower) PP_CHAIN(2, true);
+    else PP_CHAIN(2, false);
+  } else {
+    if (lower) PP_CHAIN(16, true);
+    else PP_CHAIN(16, false);
+  }
+#undef PP_CHAIN
+  PP_HIP(hipGetLastError());
+}
+
+// S^-1 = U^-1 U^-H of the factor, rounded once from extended precision
+static void invert_overlap(OverlapFactor& o) {
+  const int n = o.n, sd = o.sd;
+  auto U = [&](int i, int j) -> long double { return o.u_host[(size_t)j * (sd + 1) + sd + i - j]; };
+  std::vector<double> si((size_t)n * n);
+  std::vector<long double> x(n);
+  for (int c = 0; c < n; ++c) {
+    for (int i = 0; i < n; ++i) {  // U^-H e_c
+      long double t = i == c ? 1.0L : 0.0L;
+      for (int j = std::max(c, i - sd); j < i; ++j) t -= U(j, i) * x[j];
+      x[i] = i < c ? 0.0L : t / U(i, i);
+    }
+    for (int i = n - 1; i >= 0; --i) {  // U^-1 of it
+      long double t = x[i];
+      for (int j = i + 1; j <= std::min(n - 1, i + sd); ++j) t -= U(i, j) * x[j];
+      x[i] = t / U(i, i);
+      si[(size_t)c * n + i] = (double)x[i];
+    }
+  }
+  o.s_inv.upload(si.data(), si.size());
+  PP_HIP(hipDeviceSynchronize());  // the upload reads a host vector that goes out of scope
+}
+
 template <int SD>
 static void launch_window(int op, bool conj, const double* u, int n, long long pre, long long post, double2* data,
                           int blocks, int threads, hipStream_t s) {
 #define PP_OW(OPC, CJ) \
   hipLaunchKernelGGL((overlap_window_kernel<OPC, CJ, SD>), dim3(blocks), dim3(threads), 0, s, u, n, pre, post, data)
   switch (op) {
-    case PP_OVERLAP_MULTIPLY: PP_OW(PP_OVERLAP_MULTIPLY, false); break;
     case PP_OVERLAP_SOLVE: PP_OW(PP_OVERLAP_SOLVE, false); break;
-    case PP_OVERLAP_SQRT_MULTIPLY:
-      if (conj) PP_OW(PP_OVERLAP_SQRT_MULTIPLY, true); else PP_OW(PP_OVERLAP_SQRT_MULTIPLY, false);
-      break;
     default:
       if (conj) PP_OW(PP_OVERLAP_SQRT_SOLVE, true); else PP_OW(PP_OVERLAP_SQRT_SOLVE, false);
   }
@@ -245,7 +492,7 @@ static void launch_window(int op, bool conj, const double* u, int n, long long p
 }
 
 void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const int* extents, int rank,
-                   double2* data, hipStream_t s, double2* work) {
+                   const double2* src, double2* data, hipStream_t s, double2* work) {
   PP_REQUIRE(rank >= 0 && rank < ndim, "rank out of range");
   PP_REQUIRE(extents[rank] == ov.n, "overlap size does not match the rank extent");
   long long pre = 1, post = 1;
@@ -256,6 +503,20 @@ void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const i
   const int blocks = ceil_div(fibres, threads);
   if (blocks == 0) return;
   PP_REQUIRE(op >= 0 && op <= 3, "unknown overlap op");
+  // (512 rows of 8 superdiagonals: 53 KB of LDS with the multiply's coefficients)
+  if (ov.n <= kTileRows && (op == PP_OVERLAP_SOLVE || (op != PP_OVERLAP_SQRT_SOLVE && ov.sd <= 8))) {
+    overlap_tile(ov, op, conj, pre, post, src, data, s);
+    return;
+  }
+  if (ov.n <= kTileRows && ov.sd >= 1 && ov.sd <= 8) {
+    switch (ov.sd) {
+#define PP_CH(K) case K: overlap_chain<K>(ov, conj, pre, post, src, data, s); break;
+      PP_CH(1) PP_CH(2) PP_CH(3) PP_CH(4) PP_CH(5) PP_CH(6) PP_CH(7) PP_CH(8)
+#undef PP_CH
+    }
+    return;
+  }
+  if (src != data) vec_copy(fibres * ov.n, src, data, s);
   if (ov.sd >= 1 && ov.sd <= 8 && (op == PP_OVERLAP_MULTIPLY || op == PP_OVERLAP_SQRT_MULTIPLY)) {
     const long long total = pre * ov.n * post;
     if (!work && ov.work.count < (size_t)total) ov.work.resize(total);
@@ -341,6 +602,7 @@ extern "C" int pp_overlap_create(int n, int superdiagonals, const double* s_uppe
       o->f.sd = superdiagonals;
       band_cholesky_upper_host(n, superdiagonals, s_upper, o->f.u_host);
       o->f.u.upload(o->f.u_host.data(), o->f.u_host.size());
+      if (n <= kTileRows) invert_overlap(o->f);
       PP_HIP(hipDeviceSynchronize());
     } catch (...) {
       delete o;
@@ -365,6 +627,7 @@ extern "C" int pp_overlap_apply(const pp_overlap* ov, int op, int conj, int ndim
                                 pp_cplx* data, pp_stream stream) {
   return guarded([&] {
     PP_REQUIRE(ov && extents && data, "NULL argument");
-    overlap_apply(ov->f, op, conj != 0, ndim, extents, rank, reinterpret_cast<double2*>(data), (hipStream_t)stream);
+    double2* d = reinterpret_cast<double2*>(data);
+    overlap_apply(ov->f, op, conj != 0, ndim, extents, rank, d, d, (hipStream_t)stream);
   });
 }

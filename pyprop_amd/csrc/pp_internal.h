@@ -110,12 +110,13 @@ struct OverlapFactor {
   int sd = 0;                    // superdiagonals
   std::vector<double> u_host;    // (n, sd+1) upper band, [j][sd + i - j]
   DeviceBuffer<double> u;        // same layout on device
+  DeviceBuffer<double> s_inv;    // S^-1, dense, up to the tile kernel's rows
   mutable DeviceBuffer<double2> work;  // out-of-place passes of the multiply ops (grown on demand)
 };
-// work: out-of-place buffer of the multiply ops (as many elements as data); NULL uses ov.work,
-// grown on demand
+// data <- op src along one rank (src may be data).  Beyond the tile kernel's rows the multiply ops
+// need an out-of-place buffer: work (as many elements as data); NULL uses ov.work, grown on demand
 void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const int* extents, int rank,
-                   double2* data, hipStream_t s, double2* work = nullptr);
+                   const double2* src, double2* data, hipStream_t s, double2* work = nullptr);
 
 }  // namespace pp
 

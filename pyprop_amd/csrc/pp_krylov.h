@@ -29,7 +29,11 @@ struct Repr {
     return s;
   }
   // work: out-of-place buffer of size() elements for the multiply ops (NULL: each factor's own)
-  void overlap(int op, bool conj, double2* psi, hipStream_t s, double2* work = nullptr) const;
+  void overlap(int op, bool conj, double2* psi, hipStream_t s, double2* work = nullptr) const {
+    overlap_into(op, conj, psi, psi, s, work);
+  }
+  // dst <- op src
+  void overlap_into(int op, bool conj, const double2* src, double2* dst, hipStream_t s, double2* work = nullptr) const;
 };
 
 struct Hamiltonian {
