@@ -88,7 +88,14 @@ struct Pamp {
 
 struct Precond {
   int nchan = 0, n1 = 0, n2 = 0, b = 0;
-  // per channel c, block row I (n2 x n2 row-major blocks):
+  // Symmetric blocks (precond.hip): superblocks of b block rows, eliminated from both ends.
+  bool sym = false;
+  int ns = 0, mid = 0;          // superblocks per channel, the one where the two chains meet
+  double2 sh = {}, ss = {};
+  DeviceBuffer<double2> dinv;   // [c][s][b n2][b n2] inverse pivot blocks, upper triangle, half diagonal
+  DeviceBuffer<double> pc;      // [c][I][delta - 1][2 b + 1][n2] entries ((I, i), (I + delta, i + d - b)) of P_c
+  DeviceBuffer<double> s1, s2;  // [I][delta] and [2 b + 1][n2] bands of the overlaps
+  // Otherwise, per channel c, block row I (n2 x n2 row-major blocks):
   DeviceBuffer<double2> linv;  // [c][I]      L_II^-1 (unit lower)
   DeviceBuffer<double2> lp;    // [c][I][row][q*n2 + j] = (L_II^-1 L_{I,I-b+q})(row, j)
   DeviceBuffer<double2> uinv;  // [c][I]      U_II^-1
