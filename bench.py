@@ -536,9 +536,10 @@ def main():
         time_potgen(torch, helium_system())
         return
     sysm, repr_, psi, base = build_workload(torch)
-    nnz = sum(int(np.prod(p.source.shape)) for p in base.PotentialList)
     N = sysm.size
-    alg_bytes = 8 * nnz + 2 * 16 * N  # real float64 potential elements + src read + dst write
+    # potential values as the plan stores them (float64, repeated fibres and mirrored diagonals once)
+    # + src read + dst write
+    alg_bytes = sum(p.stream_bytes for p in base.PotentialList) + 2 * 16 * N
     dt = 0.01
     t0 = 0.5 * sysm.pulse.pulse_duration
     mv_in = matvec_input(torch, repr_, sysm.shape)

@@ -37,6 +37,7 @@ struct TPPlanDevice {
   long long n_fibres = 0;
   long long tuple_count = 0;
   int non_empty = 0;
+  int order_count = 0;  // entries of fib_order (compact plans: with -1 for none)
   int n = 0;
 };
 
@@ -44,6 +45,8 @@ struct TPTerm {
   TPGeometry geom;
   bool is_real = false;
   bool dia = false;
+  bool sym = false;                // real bands, all symmetric: diagonals d >= hb only are stored
+  std::vector<int> canon;          // stored fibre of each potential fibre (empty: itself)
   int inner_kind = 0;
   int bw = 0;
   long long pot_elements = 0;

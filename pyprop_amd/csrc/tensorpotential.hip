@@ -20,6 +20,12 @@
 //    fully coalesced loads (consecutive lanes read consecutive addresses), the source
 //    window is staged in LDS per wave.  If every imaginary part is zero the diagonals are
 //    stored as float64 (8 B/element instead of 16).  This path is HBM-bound.
+//    Real potentials are then stored once where they repeat (compact_term): a term whose bands
+//    are all symmetric keeps the diagonals d >= hb only, row i of a lower diagonal being read at
+//    row i - (hb - d) of its mirror image; fibres that are equal bit for bit are kept once.
+//    Potentials of this kind repeat a lot: (i1, j1) and (j1, i1) give the same band, and so do
+//    the angular pairs (c, c') and (c', c).  Helium (42 channels x 60 x 60): 0.49 GB kept of 2.65.
+//    The sums and their order do not change.
 //  * all other storages go through a generic per-row entry list (CSR) over the
 //    reference layout; correct for every storage, not tuned.
 #include <hip/hip_runtime.h>
@@ -28,6 +34,7 @@
 #include <array>
 #include <cstring>
 #include <numeric>
+#include <unordered_map>
 #include <vector>
 
 #include "pp_common.h"
@@ -137,23 +144,29 @@ __device__ inline void acc_scaled(C& acc, C s, C p) {
   acc.y = fma(s.y, p.x, acc.y);
 }
 
-// streaming (non-temporal) loads: the diagonals are read exactly once per product
-typedef double pp_d2v __attribute__((ext_vector_type(2)));
-typedef float pp_f2v __attribute__((ext_vector_type(2)));
-__device__ inline double ld_stream(const double* p) { return __builtin_nontemporal_load(p); }
-__device__ inline float ld_stream(const float* p) { return __builtin_nontemporal_load(p); }
-__device__ inline double2 ld_stream(const double2* p) {
-  const pp_d2v v = __builtin_nontemporal_load(reinterpret_cast<const pp_d2v*>(p));
-  return make_double2(v.x, v.y);
-}
-__device__ inline float2 ld_stream(const float2* p) {
-  const pp_f2v v = __builtin_nontemporal_load(reinterpret_cast<const pp_f2v*>(p));
-  return make_float2(v.x, v.y);
+// One value of a band through a buffer descriptor: byte offset lane_off per lane (kPastBand: masked,
+// reads zero) plus a uniform one.  KEEP: the value is read again soon; otherwise the diagonals are
+// read exactly once per product and streamed past the caches (non-temporal, bit 1 of the cache policy).
+typedef unsigned pp_u2v __attribute__((ext_vector_type(2)));
+typedef unsigned pp_u4v __attribute__((ext_vector_type(4)));
+enum { kStreamed = 0, kMixed = 1, kSymmetric = 2 };  // how a plan's terms are stored
+constexpr int kPastBand = 0x40000000;  // fibres are far smaller
+template <class V, bool KEEP>
+__device__ __forceinline__ V ld_band(__amdgpu_buffer_rsrc_t band, int lane_off, int off) {
+  constexpr int policy = KEEP ? 0 : 2;
+  if constexpr (sizeof(V) == 4) {
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(band, lane_off, off, policy));
+  } else if constexpr (sizeof(V) == 8) {
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(band, lane_off, off, policy));
+  } else {
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(band, lane_off, off, policy));
+  }
 }
 
 template <class C>
 struct DiaArgs {
-  const int4* tuples;   // {src fibre, potential fibre, (term << 1) | conj, 0}
+  const int4* tuples;   // {src fibre, stored potential fibre, (term << 1) | conj, 0}
+  unsigned sym;         // bit t: term t keeps the diagonals d >= hb only
   const int* fib_ptr;   // per destination fibre, tuple range
   const int* fib_order; // launch order
   const void* dia[kMaxTerms];
@@ -166,14 +179,20 @@ struct DiaArgs {
   int accumulate;       // dst_out = (accumulate ? dst_in : 0) + addend + alpha * sum
 };
 
-template <class V, class C, int BW, int NR>
+// COMPACT: kMixed, some term is stored compactly; kSymmetric, all are and keep half the diagonals (the
+// offsets then are the same for every tuple).  Their values are read again soon (as a mirror image, or by
+// another fibre), so they are left in the caches instead of streamed past them.  Helium's full H in
+// FP64: 428 us streaming every fibre (HBM), 172 us, bound by the L1's rate of 8-byte loads: 251 with the
+// mirror images read as well (16 clocks of a CU per load instruction).
+template <class V, class C, int BW, int NR, int COMPACT>
 __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
   constexpr int HB = (BW - 1) / 2;
   constexpr int WIN = NR * 64 + BW;
   __shared__ C xs[4][WIN];  // per-wave source window; reused for the final reduction
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int fib = a.fib_order[blockIdx.x];
+  if (fib < 0) return;
   const int t0 = a.fib_ptr[fib];
   const int cnt = a.fib_ptr[fib + 1] - t0;
   const int w0 = t0 + (int)(((long long)cnt * wave) >> 2);
@@ -184,32 +203,129 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
   C acc[NR];
 #pragma unroll
   for (int r = 0; r < NR; ++r) acc[r] = cz<C>();
+  // One row per lane and symmetric bands throughout: element (i, i + k) is used where it is read, for
+  // row i with x_{i+k} and for row i + k with lane i's own x_i.  The shift by k is the same for all
+  // tuples, so those products gather in an accumulator per k and move to their rows once, at the end:
+  // no mirror image is read, and half of the windows' LDS reads go.
+  constexpr bool SCATTER = COMPACT == kSymmetric && NR == 1;
+  constexpr int NK = SCATTER ? HB : 0;
+  C below[NK + 1];  // below[k]: to be added to row i + k
+#pragma unroll
+  for (int k = 0; k <= NK; ++k) below[k] = cz<C>();
   wave_sync();
-  for (int t = w0; t < w1; ++t) {
-    const int4 tp = a.tuples[t];
-    const C* x = a.src + (long long)tp.x * n;
+  // Lane t holds term t's potential and scale, and lane l the l-th of the next 64 tuples: reading them
+  // from memory one by one (scalar loads, whose waits are those of LDS too) stalled every tuple.
+  const int tl = min(lane, kMaxTerms - 1);
+  const unsigned long long dia_l = reinterpret_cast<unsigned long long>(a.dia[tl]);
+  const C scale_l = a.scale[tl];
+  int4 tup_l = make_int4(0, 0, 0, 0);
+  auto from_lane = [](int v, int l) { return __builtin_amdgcn_readlane(v, l); };
+  auto tuple = [&](int l) {
+    return make_int4(from_lane(tup_l.x, l), from_lane(tup_l.y, l), from_lane(tup_l.z, l), 0);
+  };
+  // a tuple's source values and its rows' bands (lanes past the fibre repeat its last row)
+  auto load = [&](const int4& tp, C (&x)[NR], V (&v)[NR][BW]) {
+    const int term = tp.z >> 1;
+    const bool sym = COMPACT == kSymmetric || (COMPACT == kMixed && (a.sym >> term & 1));
+    const C* xp = a.src + (long long)tp.x * n;
+    const unsigned long long base = (unsigned)from_lane((int)(dia_l & 0xffffffffu), term) |
+                                    (unsigned long long)(unsigned)from_lane((int)(dia_l >> 32), term) << 32;
+    const int fibre = (sym ? HB + 1 : BW) * n;  // stored values of a potential fibre
+    const __amdgpu_buffer_rsrc_t band = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void*>(base + (unsigned long long)tp.y * fibre * sizeof(V)), (short)0,
+        fibre * (int)sizeof(V), 0x00020000);
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
       const int i = lane + 64 * r;
-      if (i < n) xw[HB + i] = x[i];
+      x[r] = xp[min(i, n - 1)];
+#pragma unroll
+      for (int k = 0; k <= HB; ++k)
+#pragma unroll
+        for (int m = 0; m < (k && !SCATTER ? 2 : 1); ++m) {  // a diagonal and its mirror image, whose lines are the same
+          const int d = m ? HB - k : HB + k;
+          // stored diagonal of element (i, i + d - HB); of a mirrored one the row is i - (HB - d), and
+          // rows outside the matrix, like lanes past the fibre, are masked by an offset past the buffer
+          const int first = sym && m ? k : 0;
+          const int off = (sym ? k : d) * n - first;
+          v[r][d] =
+              ld_band<V, COMPACT != 0>(band, i < n && i >= first ? i * (int)sizeof(V) : kPastBand, off * (int)sizeof(V));
+        }
     }
-    wave_sync();
+  };
+  auto use = [&](const int4& tp, const C (&x)[NR], const V (&v)[NR][BW]) {
     const int term = tp.z >> 1;
     const bool cj = tp.z & 1;
-    const V* v = reinterpret_cast<const V*>(a.dia[term]) + (long long)tp.y * BW * n;
-    const C s = a.scale[term];
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
       const int i = lane + 64 * r;
-      if (i < n) {
-        V vv[BW];
+      if (i < n) xw[HB + i] = x[r];
+    }
+    wave_sync();
+    C s;
+    if constexpr (sizeof(C) == sizeof(double2)) {
+      s.x = __hiloint2double(from_lane(__double2hiint(scale_l.x), term), from_lane(__double2loint(scale_l.x), term));
+      s.y = __hiloint2double(from_lane(__double2hiint(scale_l.y), term), from_lane(__double2loint(scale_l.y), term));
+    } else {
+      s.x = __int_as_float(from_lane(__float_as_int(scale_l.x), term));
+      s.y = __int_as_float(from_lane(__float_as_int(scale_l.y), term));
+    }
 #pragma unroll
-        for (int d = 0; d < BW; ++d) vv[d] = ld_stream(v + d * n + i);
-        C part = cz<C>();
+    for (int r = 0; r < NR; ++r) {
+      const int i = lane + 64 * r;
+      C part = cz<C>();
+      if constexpr (SCATTER) {
+        C sx = cz<C>();
+        acc_scaled(sx, s, x[r]);
+        acc_vx(part, v[r][HB], x[r], cj);
 #pragma unroll
-        for (int d = 0; d < BW; ++d) acc_vx(part, vv[d], xw[i + d], cj);
-        acc_scaled(acc[r], s, part);
+        for (int k = 1; k <= NK; ++k) {
+          acc_vx(part, v[r][HB + k], xw[i + HB + k], cj);
+          acc_vx(below[k], v[r][HB + k], sx, cj);
+        }
+      } else {
+#pragma unroll
+        for (int d = 0; d < BW; ++d) acc_vx(part, v[r][d], xw[i + d], cj);
       }
+      acc_scaled(acc[r], s, part);
+    }
+    wave_sync();
+  };
+  for (int b0 = w0; b0 < w1; b0 += 64) {
+    const int last = min(64, w1 - b0) - 1;
+    tup_l = a.tuples[b0 + min(lane, last)];
+    if constexpr (NR * BW * sizeof(V) <= 13 * sizeof(double)) {
+      // the next tuple's loads are issued before the current one is used: a wave waits for memory about
+      // half as often, for one more set of registers
+      C xa[NR], xb[NR];
+      V va[NR][BW], vb[NR][BW];
+      int4 ta = tuple(0), tb;
+      load(ta, xa, va);
+      for (int l = 0; l <= last; l += 2) {
+        tb = tuple(min(l + 1, last));
+        load(tb, xb, vb);
+        use(ta, xa, va);
+        if (l + 1 > last) break;
+        ta = tuple(min(l + 2, last));
+        load(ta, xa, va);
+        use(tb, xb, vb);
+      }
+    } else {
+      C x[NR];
+      V v[NR][BW];
+      for (int l = 0; l <= last; ++l) {
+        const int4 tp = tuple(l);
+        load(tp, x, v);
+        use(tp, x, v);
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 1; k <= NK; ++k) {
+    xw[lane] = below[k];
+    wave_sync();
+    if (lane >= k) {
+      acc[0].x += xw[lane - k].x;
+      acc[0].y += xw[lane - k].y;
     }
     wave_sync();
   }
@@ -351,6 +467,7 @@ __global__ __launch_bounds__(256) void expand_terms_kernel(long long p0, long lo
     double v = 0.0;
 #pragma unroll
     for (int t = 0; t < T; ++t) v = fma(coeffs[t * p0 + a], R[t], v);
+    typedef double pp_d2v __attribute__((ext_vector_type(2)));
     pp_d2v* o = reinterpret_cast<pp_d2v*>(out + a * rc + r);
     pp_d2v w = {v, 0.0};
     if (accumulate) w += *o;
@@ -467,6 +584,45 @@ static void build_inner_csr(const TPGeometry& g, std::vector<int>& row_ptr, std:
   for (auto& r : rows) entries.insert(entries.end(), r.begin(), r.end());
 }
 
+static unsigned symmetric_terms(const std::vector<const TPTerm*>& terms) {
+  unsigned m = 0;
+  for (size_t t = 0; t < terms.size(); ++t) m |= (terms[t]->sym ? 1u : 0u) << t;
+  return m;
+}
+static bool any_compact(const std::vector<const TPTerm*>& terms) {
+  for (auto* t : terms)
+    if (t->sym || !t->canon.empty()) return true;
+  return false;
+}
+
+// Launch order of a compact plan: workgroup b runs on XCD b % 8, and the destination fibres (.., i) and
+// (.., j) of one group (equal indices but the last outer one) read the same stored fibres at about
+// the same time.  Each XCD therefore takes a contiguous range of fibres of about an eighth of the
+// tuples, heaviest groups first, so that a stored fibre comes into its L2 once; ranges that are
+// shorter in number are filled up with -1.  Helium's full H: longest fibres first 203 us, this order
+// 181 us.
+static void xcd_order(TPPlanData& pd, int group) {
+  constexpr int kXcds = 8;
+  auto count = [&](long long f) { return pd.fib_ptr[f + 1] - pd.fib_ptr[f]; };
+  std::vector<int> weight((pd.n_fibres + group - 1) / group, 0);
+  for (long long f = 0; f < pd.n_fibres; ++f) weight[f / group] = std::max(weight[f / group], count(f));
+  std::vector<int> part[kXcds];
+  const long long total = pd.fib_ptr[pd.n_fibres] + pd.n_fibres;  // an empty fibre is some work too
+  long long done = 0;
+  for (long long f = 0; f < pd.n_fibres; ++f) {
+    part[std::min<long long>(kXcds - 1, done * kXcds / total)].push_back((int)f);
+    done += count(f) + 1;
+  }
+  size_t most = 0;
+  for (auto& p : part) {
+    std::stable_sort(p.begin(), p.end(), [&](int a, int b) { return weight[a / group] > weight[b / group]; });
+    most = std::max(most, p.size());
+  }
+  pd.fib_order.assign(most * kXcds, -1);
+  for (int x = 0; x < kXcds; ++x)
+    for (size_t k = 0; k < part[x].size(); ++k) pd.fib_order[k * kXcds + x] = part[x][k];
+}
+
 TPPlanData build_plan_host(const std::vector<const TPTerm*>& terms) {
   PP_REQUIRE(!terms.empty() && terms.size() <= (size_t)kMaxTerms, "1..8 terms per plan");
   const TPGeometry& g0 = terms[0]->geom;
@@ -482,8 +638,9 @@ TPPlanData build_plan_host(const std::vector<const TPTerm*>& terms) {
     PP_REQUIRE(g.rank == R, "terms must share the rank");
     for (int r = 0; r < R; ++r) PP_REQUIRE(g.src_ext[r] == g0.src_ext[r], "terms must share the source shape");
     const bool ignore_conj = g.ids[R - 1] == PP_STORAGE_BAND;  // zhbmv takes no conjugate flag
+    const std::vector<int>& canon = terms[t]->canon;
     for (const Tuple& tp : outer_tuples(g))
-      byfib[tp.dst].push_back(make_int4(tp.src, tp.pot, (int)(t << 1) | (ignore_conj ? 0 : tp.conj), 0));
+      byfib[tp.dst].push_back(make_int4(tp.src, canon.empty() ? tp.pot : canon[tp.pot], (int)(t << 1) | (ignore_conj ? 0 : tp.conj), 0));
   }
   pd.fib_ptr.assign(nf + 1, 0);
   for (long long f = 0; f < nf; ++f) pd.fib_ptr[f + 1] = pd.fib_ptr[f] + (int)byfib[f].size();
@@ -497,6 +654,7 @@ TPPlanData build_plan_host(const std::vector<const TPTerm*>& terms) {
   pd.non_empty = 0;
   for (long long f = 0; f < nf; ++f)
     if (pd.fib_ptr[f + 1] > pd.fib_ptr[f]) ++pd.non_empty;
+  if (any_compact(terms)) xcd_order(pd, R > 1 ? g0.src_ext[R - 2] : 1);
   return pd;
 }
 
@@ -507,14 +665,138 @@ void upload_plan(const TPPlanData& pd, TPPlanDevice& dv, hipStream_t s) {
   dv.n = pd.n;
   dv.n_fibres = pd.n_fibres;
   dv.non_empty = pd.non_empty;
+  dv.order_count = (int)pd.fib_order.size();
   dv.tuple_count = (long long)pd.tuples.size();
+}
+
+// flag |= some element (i, i + d - hb) below the diagonal differs in its bits from its mirror image
+__global__ void asymmetric_kernel(const double* __restrict__ dia, long long fibres, int n, int bw,
+                                  unsigned long long* flag) {
+  const int hb = (bw - 1) / 2;
+  const long long total = fibres * hb * (long long)n;
+  bool differs = false;
+  for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
+       idx += (long long)gridDim.x * blockDim.x) {
+    const int i = (int)(idx % n), d = (int)(idx / n % hb), j = i + d - hb;
+    const double* f = dia + idx / ((long long)n * hb) * bw * n;
+    if (j >= 0) differs |= __double_as_longlong(f[d * n + i]) != __double_as_longlong(f[(2 * hb - d) * n + j]);
+  }
+  if (__any(differs) && (threadIdx.x & 63) == 0) atomicOr(flag, 1ull);
+}
+
+// hash[f] of the bits of rows [first, first + len) of fibre f: one wave per fibre, a sum over its
+// values of a multiplicative mix of (bits, position)
+__global__ __launch_bounds__(256) void fibre_hash_kernel(const double* __restrict__ dia, long long fibres, int stride,
+                                                         int first, int len, unsigned long long* __restrict__ hash) {
+  const long long f = blockIdx.x * 4LL + (threadIdx.x >> 6);
+  if (f >= fibres) return;
+  const double* v = dia + f * stride + first;
+  unsigned long long h = 0;
+  for (int k = threadIdx.x & 63; k < len; k += 64) {
+    unsigned long long w = (unsigned long long)__double_as_longlong(v[k]) + 0x9E3779B97F4A7C15ull * (k + 1);
+    w = (w ^ (w >> 30)) * 0xBF58476D1CE4E5B9ull;
+    w = (w ^ (w >> 27)) * 0x94D049BB133111EBull;
+    h += w ^ (w >> 31);
+  }
+  for (int off = 32; off > 0; off >>= 1) h += __shfl_down(h, off, 64);
+  if ((threadIdx.x & 63) == 0) hash[f] = h;
+}
+
+// flag |= fibre f differs in its bits from fibre rep[f]
+__global__ __launch_bounds__(256) void fibre_differs_kernel(const double* __restrict__ dia, long long fibres, int stride,
+                                                            int first, int len, const int* __restrict__ rep,
+                                                            unsigned long long* flag) {
+  const long long f = blockIdx.x * 4LL + (threadIdx.x >> 6);
+  if (f >= fibres || rep[f] == f) return;
+  const double *a = dia + f * stride + first, *b = dia + (long long)rep[f] * stride + first;
+  bool differs = false;
+  for (int k = threadIdx.x & 63; k < len; k += 64) differs |= __double_as_longlong(a[k]) != __double_as_longlong(b[k]);
+  if (__any(differs) && (threadIdx.x & 63) == 0) atomicOr(flag, 1ull);
+}
+
+// out[u] = rows [first, first + len) of fibre kept[u]
+__global__ __launch_bounds__(256) void gather_fibres_kernel(const double* __restrict__ dia, long long kept_count,
+                                                            int stride, int first, int len,
+                                                            const int* __restrict__ kept, double* __restrict__ out) {
+  const long long u = blockIdx.x * 4LL + (threadIdx.x >> 6);
+  if (u >= kept_count) return;
+  const double* v = dia + (long long)kept[u] * stride + first;
+  for (int k = threadIdx.x & 63; k < len; k += 64) out[u * len + k] = v[k];
+}
+
+// Stores a real banded term compactly where that saves at least a quarter (a hash collision keeps it
+// as it is: equality is checked value by value).
+static void compact_term(TPTerm& term, long long pfib, int n, hipStream_t s) {
+  if (pfib >= (1ll << 31)) return;
+  const int bw = term.bw, hb = (bw - 1) / 2, stride = bw * n;
+  const int wave_blocks = ceil_div(pfib, 4);
+  DeviceBuffer<unsigned long long> flag(1), hash(pfib);
+  auto read_flag = [&]() {
+    unsigned long long h = 0;
+    PP_HIP(hipMemcpyAsync(&h, flag.ptr, sizeof(h), hipMemcpyDeviceToHost, s));
+    PP_HIP(hipStreamSynchronize(s));
+    return h != 0;
+  };
+  bool sym = hb > 0;
+  if (sym) {
+    PP_HIP(hipMemsetAsync(flag.ptr, 0, sizeof(unsigned long long), s));
+    const long long total = pfib * hb * (long long)n;
+    hipLaunchKernelGGL(asymmetric_kernel, dim3((int)std::min<long long>(65536, (total + 255) / 256)), dim3(256), 0, s,
+                       term.dia_real.ptr, pfib, n, bw, flag.ptr);
+    PP_HIP(hipGetLastError());
+    sym = !read_flag();
+  }
+  const int first = sym ? hb * n : 0, len = sym ? (hb + 1) * n : stride;
+  hipLaunchKernelGGL(fibre_hash_kernel, dim3(wave_blocks), dim3(256), 0, s, term.dia_real.ptr, pfib, stride, first, len,
+                     hash.ptr);
+  PP_HIP(hipGetLastError());
+  std::vector<unsigned long long> h(pfib);
+  PP_HIP(hipMemcpyAsync(h.data(), hash.ptr, pfib * sizeof(h[0]), hipMemcpyDeviceToHost, s));
+  PP_HIP(hipStreamSynchronize(s));
+  std::unordered_map<unsigned long long, int> seen;
+  seen.reserve(pfib);
+  std::vector<int> canon(pfib), rep(pfib), kept;
+  for (long long f = 0; f < pfib; ++f) {
+    const auto it = seen.emplace(h[f], (int)kept.size());
+    if (it.second) kept.push_back((int)f);
+    canon[f] = it.first->second;
+    rep[f] = kept[canon[f]];
+  }
+  bool merged = kept.size() < (size_t)pfib;
+  if (merged) {
+    DeviceBuffer<int> reps;
+    reps.upload(rep.data(), rep.size(), s);
+    PP_HIP(hipMemsetAsync(flag.ptr, 0, sizeof(unsigned long long), s));
+    hipLaunchKernelGGL(fibre_differs_kernel, dim3(wave_blocks), dim3(256), 0, s, term.dia_real.ptr, pfib, stride, first,
+                       len, reps.ptr, flag.ptr);
+    PP_HIP(hipGetLastError());
+    if (read_flag()) merged = false;
+  }
+  if (!merged) {
+    kept.resize(pfib);
+    std::iota(kept.begin(), kept.end(), 0);
+  }
+  const long long size = (long long)kept.size() * len;
+  if (size * 4 > pfib * (long long)stride * 3) return;
+  DeviceBuffer<int> keep;
+  keep.upload(kept.data(), kept.size(), s);
+  DeviceBuffer<double> out(size);
+  hipLaunchKernelGGL(gather_fibres_kernel, dim3(ceil_div((long long)kept.size(), 4)), dim3(256), 0, s,
+                     term.dia_real.ptr, (long long)kept.size(), stride, first, len, keep.ptr, out.ptr);
+  PP_HIP(hipGetLastError());
+  PP_HIP(hipStreamSynchronize(s));  // before the buffers that the copy reads are released
+  std::swap(term.dia_real.ptr, out.ptr);
+  std::swap(term.dia_real.count, out.count);
+  term.sym = sym;
+  if (merged) term.canon = std::move(canon);
+  term.stream_bytes = size * (long long)sizeof(double);
 }
 
 static bool is_band(int id) { return id == PP_STORAGE_BANDNH || id == PP_STORAGE_BAND; }
 
 void tp_create_impl(int rank, const int* ids, const double2* potential, const int* pot_ext,
                     const int* src_ext, const int32_t* const* pairs, const int* pair_counts,
-                    hipStream_t s, TPTerm& term) {
+                    hipStream_t s, TPTerm& term, bool compact) {
   PP_REQUIRE(rank >= 1 && rank <= kMaxRank, "rank must be 1..4");
   PP_REQUIRE(potential != nullptr, "potential is NULL");
   TPGeometry& g = term.geom;
@@ -578,6 +860,7 @@ void tp_create_impl(int rank, const int* ids, const double2* potential, const in
       term.stream_bytes = total * (long long)sizeof(double2);
     }
     PP_HIP(hipGetLastError());
+    if (compact && term.is_real) compact_term(term, pfib, n, s);
   } else {
     term.dia = false;
     term.vref.resize(pcount);
@@ -597,7 +880,7 @@ void tp_create_impl(int rank, const int* ids, const double2* potential, const in
 void tp_ensure_f32(const TPTerm& t, hipStream_t s) {
   if (!t.dia) throw Error(PP_ERR_INVALID, "FP32 multiply needs a banded innermost storage");
   TPTerm& m = const_cast<TPTerm&>(t);
-  const long long total = t.pot_fibres * t.bw * (long long)t.plan.n;
+  const long long total = (long long)(t.is_real ? t.dia_real.count : t.dia_cplx.count);  // as stored
   if (t.is_real) {
     if (m.dia_real_f.count == (size_t)total) return;
     m.dia_real_f.resize(total);
@@ -618,30 +901,30 @@ void tp_ensure_f32(const TPTerm& t, hipStream_t s) {
 // ----------------------------------------------------------------------------------
 // launch
 // ----------------------------------------------------------------------------------
-template <class V, class C, int BW>
+template <class V, class C, int BW, int COMPACT>
 static void launch_dia_bw(const DiaArgs<C>& a, int nr, int blocks, hipStream_t s) {
   // rows per lane rounded up to 1, 2, 4 or 8 (the kernel masks rows >= n)
-  if (nr <= 1) hipLaunchKernelGGL((tp_dia_kernel<V, C, BW, 1>), dim3(blocks), dim3(256), 0, s, a);
-  else if (nr <= 2) hipLaunchKernelGGL((tp_dia_kernel<V, C, BW, 2>), dim3(blocks), dim3(256), 0, s, a);
-  else if (nr <= 4) hipLaunchKernelGGL((tp_dia_kernel<V, C, BW, 4>), dim3(blocks), dim3(256), 0, s, a);
-  else if (nr <= 8) hipLaunchKernelGGL((tp_dia_kernel<V, C, BW, 8>), dim3(blocks), dim3(256), 0, s, a);
+  if (nr <= 1) hipLaunchKernelGGL((tp_dia_kernel<V, C, BW, 1, COMPACT>), dim3(blocks), dim3(256), 0, s, a);
+  else if (nr <= 2) hipLaunchKernelGGL((tp_dia_kernel<V, C, BW, 2, COMPACT>), dim3(blocks), dim3(256), 0, s, a);
+  else if (nr <= 4) hipLaunchKernelGGL((tp_dia_kernel<V, C, BW, 4, COMPACT>), dim3(blocks), dim3(256), 0, s, a);
+  else if (nr <= 8) hipLaunchKernelGGL((tp_dia_kernel<V, C, BW, 8, COMPACT>), dim3(blocks), dim3(256), 0, s, a);
   else throw Error(PP_ERR_INVALID, "innermost extent too large for the banded kernel");
 }
 
-template <class V, class C>
+template <class V, class C, int COMPACT>
 static void launch_dia(const DiaArgs<C>& a, int bw, int nr, int blocks, hipStream_t s) {
   switch (bw) {
-    case 1: launch_dia_bw<V, C, 1>(a, nr, blocks, s); break;
-    case 3: launch_dia_bw<V, C, 3>(a, nr, blocks, s); break;
-    case 5: launch_dia_bw<V, C, 5>(a, nr, blocks, s); break;
-    case 7: launch_dia_bw<V, C, 7>(a, nr, blocks, s); break;
-    case 9: launch_dia_bw<V, C, 9>(a, nr, blocks, s); break;
-    case 11: launch_dia_bw<V, C, 11>(a, nr, blocks, s); break;
-    case 13: launch_dia_bw<V, C, 13>(a, nr, blocks, s); break;
-    case 15: launch_dia_bw<V, C, 15>(a, nr, blocks, s); break;
-    case 17: launch_dia_bw<V, C, 17>(a, nr, blocks, s); break;
-    case 19: launch_dia_bw<V, C, 19>(a, nr, blocks, s); break;
-    case 21: launch_dia_bw<V, C, 21>(a, nr, blocks, s); break;
+    case 1: launch_dia_bw<V, C, 1, COMPACT>(a, nr, blocks, s); break;
+    case 3: launch_dia_bw<V, C, 3, COMPACT>(a, nr, blocks, s); break;
+    case 5: launch_dia_bw<V, C, 5, COMPACT>(a, nr, blocks, s); break;
+    case 7: launch_dia_bw<V, C, 7, COMPACT>(a, nr, blocks, s); break;
+    case 9: launch_dia_bw<V, C, 9, COMPACT>(a, nr, blocks, s); break;
+    case 11: launch_dia_bw<V, C, 11, COMPACT>(a, nr, blocks, s); break;
+    case 13: launch_dia_bw<V, C, 13, COMPACT>(a, nr, blocks, s); break;
+    case 15: launch_dia_bw<V, C, 15, COMPACT>(a, nr, blocks, s); break;
+    case 17: launch_dia_bw<V, C, 17, COMPACT>(a, nr, blocks, s); break;
+    case 19: launch_dia_bw<V, C, 19, COMPACT>(a, nr, blocks, s); break;
+    case 21: launch_dia_bw<V, C, 21, COMPACT>(a, nr, blocks, s); break;
     default: throw Error(PP_ERR_INVALID, "band width not instantiated (odd 1..21 supported)");
   }
 }
@@ -661,11 +944,18 @@ bool terms_fusable(const std::vector<const TPTerm*>& terms) {
   return true;
 }
 
+// Workgroups of a multiply; only the fibres with tuples need one where the others keep their value
+// (a streaming plan has those first)
+static int plan_blocks(const TPPlanDevice& plan, const std::vector<const TPTerm*>& terms, bool keeps_empty) {
+  if (any_compact(terms)) return plan.tuple_count == 0 && keeps_empty ? 0 : plan.order_count;
+  return keeps_empty ? plan.non_empty : (int)plan.n_fibres;
+}
+
 void tp_run_f64(const TPPlanDevice& plan, const std::vector<const TPTerm*>& terms,
                 const double2* scales, const double2* src, double2* dst, const double2* addend,
                 double2 alpha, bool accumulate, hipStream_t s) {
   const TPTerm* t0 = terms[0];
-  const int blocks = (accumulate && !addend) ? plan.non_empty : (int)plan.n_fibres;
+  const int blocks = plan_blocks(plan, terms, accumulate && !addend);
   if (blocks == 0) return;
   if (t0->dia) {
     DiaArgs<double2> a{};
@@ -683,8 +973,11 @@ void tp_run_f64(const TPPlanDevice& plan, const std::vector<const TPTerm*>& term
     a.alpha = alpha;
     a.accumulate = accumulate ? 1 : 0;
     const int nr = (plan.n + 63) / 64;
-    if (t0->is_real) launch_dia<double, double2>(a, t0->bw, nr, blocks, s);
-    else launch_dia<double2, double2>(a, t0->bw, nr, blocks, s);
+    a.sym = symmetric_terms(terms);
+    if (!t0->is_real) launch_dia<double2, double2, kStreamed>(a, t0->bw, nr, blocks, s);
+    else if (a.sym == (1u << terms.size()) - 1) launch_dia<double, double2, kSymmetric>(a, t0->bw, nr, blocks, s);
+  else if (any_compact(terms)) launch_dia<double, double2, kMixed>(a, t0->bw, nr, blocks, s);
+    else launch_dia<double, double2, kStreamed>(a, t0->bw, nr, blocks, s);
   } else {
     GenArgs<double2> a{};
     a.tuples = plan.tuples.ptr;
@@ -714,7 +1007,7 @@ void tp_run_f32(const TPPlanDevice& plan, const std::vector<const TPTerm*>& term
   const TPTerm* t0 = terms[0];
   PP_REQUIRE(t0->dia, "FP32 multiply needs a banded innermost storage");
   for (auto* t : terms) tp_ensure_f32(*t, s);
-  const int blocks = (accumulate && !addend) ? plan.non_empty : (int)plan.n_fibres;
+  const int blocks = plan_blocks(plan, terms, accumulate && !addend);
   if (blocks == 0) return;
   DiaArgs<float2> a{};
   a.tuples = plan.tuples.ptr;
@@ -731,8 +1024,11 @@ void tp_run_f32(const TPPlanDevice& plan, const std::vector<const TPTerm*>& term
   a.alpha = alpha;
   a.accumulate = accumulate ? 1 : 0;
   const int nr = (plan.n + 63) / 64;
-  if (t0->is_real) launch_dia<float, float2>(a, t0->bw, nr, blocks, s);
-  else launch_dia<float2, float2>(a, t0->bw, nr, blocks, s);
+  a.sym = symmetric_terms(terms);
+  if (!t0->is_real) launch_dia<float2, float2, kStreamed>(a, t0->bw, nr, blocks, s);
+  else if (a.sym == (1u << terms.size()) - 1) launch_dia<float, float2, kSymmetric>(a, t0->bw, nr, blocks, s);
+  else if (any_compact(terms)) launch_dia<float, float2, kMixed>(a, t0->bw, nr, blocks, s);
+  else launch_dia<float, float2, kStreamed>(a, t0->bw, nr, blocks, s);
   PP_HIP(hipGetLastError());
 }
 
@@ -752,7 +1048,7 @@ extern "C" int pp_tp_create(int rank, const int* storage_ids, const pp_cplx* pot
     auto* t = new pp_tensor_potential();
     try {
       tp_create_impl(rank, storage_ids, reinterpret_cast<const double2*>(potential), potential_extents,
-                     source_extents, pairs, pair_counts, (hipStream_t)stream, t->term);
+                     source_extents, pairs, pair_counts, (hipStream_t)stream, t->term, true);
     } catch (...) {
       delete t;
       throw;
@@ -808,7 +1104,7 @@ extern "C" int pp_tensor_potential_multiply(int rank, const int* storage_ids, co
       PP_REQUIRE(dest_extents[r] == source_extents[r], "dest and source extents must match");
     pp_tensor_potential t;
     tp_create_impl(rank, storage_ids, reinterpret_cast<const double2*>(potential), potential_extents,
-                   source_extents, pairs, pair_counts, (hipStream_t)stream, t.term);
+                   source_extents, pairs, pair_counts, (hipStream_t)stream, t.term, false);
     double2 sc = make_double2(scaling, 0.0);
     tp_run_f64(t.term.plan, {&t.term}, &sc, reinterpret_cast<const double2*>(source),
                reinterpret_cast<double2*>(dest), nullptr, make_double2(1.0, 0.0), true, (hipStream_t)stream);

@@ -1,0 +1,107 @@
+"""GPU tests of potentials that the multiply plan stores compactly (symmetric bands kept as half their
+diagonals, equal fibres kept once) against a dense product: all, some or none of a Hamiltonian's terms
+compact, row counts below, at and above a wave, every band width the kernel has."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+    assert t.cuda.is_available(), "GPU tests need a HIP device"
+    from pyprop_amd import _native
+    _native.load()
+    return t
+
+
+def _potential(rng, nc, n1, b1, n2, b2, kind):
+    """(TensorPotentialData, dense (nc n1 n2)^2 matrix); kind "symmetric" in every rank, "half" only in
+    the innermost, "none"."""
+    from pyprop_amd.geometry import Geometry
+    from pyprop_amd.systems import TensorPotentialData
+    p0 = np.array([(a, b) for a in range(nc) for b in range(nc)], dtype=np.int32)
+    p1 = np.array([(a, b) for a in range(n1) for b in range(max(0, a - b1), min(n1, a + b1 + 1))], dtype=np.int32)
+    w = 2 * b2 + 1
+    full = rng.standard_normal((nc, nc, n1, n1, n2, n2))
+    if kind != "none":
+        full = full + full.swapaxes(4, 5)
+    if kind == "symmetric":
+        full = full + full.swapaxes(0, 1)
+        full = full + full.swapaxes(2, 3)
+    keep1 = np.abs(np.subtract.outer(np.arange(n1), np.arange(n1))) <= b1
+    keep2 = np.abs(np.subtract.outer(np.arange(n2), np.arange(n2))) <= b2
+    full = full * keep1[None, None, :, :, None, None] * keep2
+    data = np.zeros((len(p0), len(p1), n2 * w), complex)
+    pairs2 = np.zeros((n2 * w, 2), dtype=np.int32)
+    for j in range(n2):
+        for i in range(max(0, j - b2), min(n2, j + b2 + 1)):
+            k = j * w + b2 + i - j
+            pairs2[k] = (i, j)
+            data[:, :, k] = full[p0[:, 0][:, None], p0[:, 1][:, None], p1[:, 0][None], p1[:, 1][None], i, j]
+    geo = [Geometry("Simp", p0, False, nc), Geometry("Simp", p1, True, n1), Geometry("BandNH", pairs2, True, n2)]
+    dense = full.transpose(0, 2, 4, 1, 3, 5).reshape(nc * n1 * n2, nc * n1 * n2)
+    return TensorPotentialData(kind, geo, data), dense
+
+
+@pytest.mark.parametrize("kinds", [("symmetric",), ("half",), ("none",), ("symmetric", "half"), ("symmetric", "none"),
+                                   ("none", "half", "symmetric")], ids="+".join)
+@pytest.mark.parametrize("n2,b2", [(3, 1), (13, 4), (63, 6), (64, 6), (65, 6), (130, 2), (300, 3)])
+def test_hamiltonian_of_compact_terms(torch, kinds, n2, b2):
+    from pyprop_amd.propagator import BasisPropagator, CombinedRepresentation, Wavefunction
+    rng = np.random.default_rng(n2 + len(kinds))
+    nc, n1, b1 = 3, 4, 2
+    made = [_potential(rng, nc, n1, b1, n2, b2, k) for k in kinds]
+    repr_ = CombinedRepresentation((nc, n1, n2), [None, None, None])
+    x = rng.standard_normal((nc, n1, n2)) + 1j * rng.standard_normal((nc, n1, n2))
+    psi = Wavefunction(repr_, x)
+    base = BasisPropagator(psi, [m[0] for m in made], consolidate=False)
+    out = Wavefunction(repr_)
+    base.MultiplyHamiltonianNoOverlap(psi, out, 0.0)
+    M = sum(m[1] for m in made)
+    ref = (M @ x.ravel()).reshape(x.shape)
+    bound = 2.0 ** -53 * (nc * (2 * b1 + 1) * (2 * b2 + 1) * len(kinds) + 4) * (np.abs(M) @ np.abs(x.ravel()))
+    assert np.all(np.abs(out.numpy().ravel() - ref.ravel()) <= 2 * bound)
+    # stored bytes: half the diagonals of symmetric bands, and of equal fibres one
+    for p, k in zip(base.PotentialList, kinds):
+        full = 8 * nc * nc * p.GeometryList[1].pair_count * (2 * b2 + 1) * n2
+        assert p.stream_bytes == full if k == "none" else p.stream_bytes < 0.76 * full
+    # one potential at a time, added to what is there
+    for (data, dense), p in zip(made, base.PotentialList):
+        acc = torch.ones_like(psi.data)
+        p.MultiplyPotential(psi, acc, 0.0)
+        r = (dense @ x.ravel()).reshape(x.shape) + 1.0
+        assert np.linalg.norm(acc.cpu().numpy() - r) < 1e-14 * np.linalg.norm(r)
+
+
+@pytest.mark.parametrize("n2,b2", [(13, 4), (64, 6), (100, 3)])
+def test_fp32_multiply_of_compact_terms(torch, n2, b2):
+    import ctypes as C
+    from pyprop_amd import _native as N, device as D
+    from pyprop_amd.tensorpotential import TensorPotential
+    rng = np.random.default_rng(n2)
+    data, dense = _potential(rng, 2, 4, 2, n2, b2, "symmetric")
+    p = TensorPotential(data, (2, 4, n2))
+    p.SetupStep()
+    x = rng.standard_normal((2, 4, n2)) + 1j * rng.standard_normal((2, 4, n2))
+    src = torch.from_numpy(x).to("cuda").to(torch.complex64)
+    dst = torch.zeros_like(src)
+    N.check(N.load().pp_tp_multiply_f32(p.plan, C.c_float(1.0), D.ptr(src), D.ptr(dst), D.stream_handle()))
+    ref = dense @ x.ravel()
+    assert np.linalg.norm(dst.cpu().numpy().ravel() - ref) < 1e-6 * np.linalg.norm(ref)
+
+
+def test_nan_stays_in_the_rows_it_couples_to(torch):
+    """A NaN of row j reaches rows j - b .. j + b of the innermost rank, as in the banded product."""
+    from pyprop_amd.propagator import BasisPropagator, CombinedRepresentation, Wavefunction
+    rng = np.random.default_rng(1)
+    for n2 in (40, 90):
+        data, _ = _potential(rng, 1, 1, 0, n2, 3, "symmetric")
+        repr_ = CombinedRepresentation((1, 1, n2), [None, None, None])
+        x = np.ones((1, 1, n2), complex)
+        x[0, 0, 20] = np.nan
+        psi, out = Wavefunction(repr_, x), Wavefunction(repr_)
+        BasisPropagator(psi, [data], consolidate=False).MultiplyHamiltonianNoOverlap(psi, out, 0.0)
+        bad = np.isnan(out.numpy()[0, 0].real)
+        assert np.array_equal(np.nonzero(bad)[0], np.arange(17, 24))
