@@ -292,10 +292,21 @@ __global__ void pamp_orth_check_kernel(const double2* orig2, const double2* resi
 
 // scaling-and-squaring Pade exponential of A = -i dt H (pamp.h:430-565), one workgroup.
 // work: 6 m*m matrices; out_col[i] = E(i, 0); sc[2] = E(m-1, 0).
-__global__ __launch_bounds__(256) void pade_exp_kernel(const double2* __restrict__ Hm, int m, double2 dt, int order,
+// The work matrices are in LDS when they fit (IN_LDS, m <= kPadeLds: 60 KB), for every entry of some 25
+// products and an LU is read m times over with a barrier after each: 183 us at m = 20 from memory, with
+// serial scans for the scaling and the pivots; 100 us now.
+constexpr int kPadeLds = 25;
+template <bool IN_LDS>
+__global__ __launch_bounds__(512) void pade_exp_kernel(const double2* __restrict__ Hm, int m, double2 dt, int order,
                                                         double2* __restrict__ work, double2* __restrict__ out_col,
                                                         double2* __restrict__ sc, int* __restrict__ piv_ws) {
-  pade_exp_wg(Hm, m, dt, order, work, out_col, sc + 2, piv_ws);
+  extern __shared__ double2 pade_lds[];
+  if constexpr (IN_LDS) {
+    __shared__ int piv[kPadeLds];
+    pade_exp_wg(Hm, m, dt, order, pade_lds, out_col, sc + 2, piv);
+  } else {
+    pade_exp_wg(Hm, m, dt, order, work, out_col, sc + 2, piv_ws);
+  }
 }
 
 // EigenvectorExponential (pamp.h:567-608): exp(A) ~ V diag(exp(w)) V^H with the unit-norm
@@ -477,8 +488,12 @@ void Pamp::propagate(pp_operator_fn op, void* ctx, double2* v, double2 dt, hipSt
     PP_HIP(hipMemcpyAsync(sc.ptr + 2, &c[m - 1], sizeof(double2), hipMemcpyHostToDevice, s));
     PP_HIP(hipStreamSynchronize(s));  // the host vector is released on return
   } else {
-    hipLaunchKernelGGL(pade_exp_kernel, dim3(1), dim3(256), 0, s, H.ptr, m, dt, order, work.ptr, expcol.ptr, sc.ptr,
-                       piv.ptr);
+    if (m <= kPadeLds)
+      hipLaunchKernelGGL(pade_exp_kernel<true>, dim3(1), dim3(512), 6 * m * m * sizeof(double2), s, H.ptr, m, dt, order,
+                         work.ptr, expcol.ptr, sc.ptr, piv.ptr);
+    else
+      hipLaunchKernelGGL(pade_exp_kernel<false>, dim3(1), dim3(512), 0, s, H.ptr, m, dt, order, work.ptr, expcol.ptr,
+                         sc.ptr, piv.ptr);
   }
   PP_HIP(hipGetLastError());
   // input = norm * V exp(H)[:, 0]

@@ -20,7 +20,7 @@ __device__ inline void pade_exp_wg(const double2* __restrict__ Hm, int m, double
   double2* Q = work + 3 * mm;
   double2* T = work + 4 * mm;
   double2* E = work + 5 * mm;
-  __shared__ double smax[1024];
+  __shared__ double smax[16];
   __shared__ double coeff[32];
   __shared__ int s_scale;
   const double2 f = make_double2(dt.y, -dt.x);  // -i * dt
@@ -30,11 +30,13 @@ __device__ inline void pade_exp_wg(const double2* __restrict__ Hm, int m, double
     A[i] = a;
     mx = fmax(mx, sqrt(a.x * a.x + a.y * a.y));
   }
-  smax[threadIdx.x] = mx;
+  // (a maximum: any order gives the same)
+  for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
+  if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = mx;
   __syncthreads();
   if (threadIdx.x == 0) {
     double v = 0;
-    for (int i = 0; i < (int)blockDim.x; ++i) v = fmax(v, smax[i]);
+    for (int i = 0; i < (int)(blockDim.x + 63) / 64; ++i) v = fmax(v, smax[i]);
     int s = (v > 0) ? (int)ceil(log2(v)) : 0;
     s_scale = s > 0 ? s : 0;
     coeff[0] = 1.0;
@@ -49,6 +51,7 @@ __device__ inline void pade_exp_wg(const double2* __restrict__ Hm, int m, double
     for (int idx = threadIdx.x; idx < mm; idx += blockDim.x) {
       const int row = idx % m, col = idx / m;
       double2 acc = make_double2(0, 0);
+#pragma unroll 4
       for (int k = 0; k < m; ++k) cfma(acc, X[k * m + row], Y[col * m + k]);
       C[idx] = acc;
     }
@@ -84,14 +87,21 @@ __device__ inline void pade_exp_wg(const double2* __restrict__ Hm, int m, double
   __syncthreads();
   // LU with partial pivoting (zgetrf: pivot by |re| + |im|), then solve Q X = P (zgetrs)
   for (int k = 0; k < m; ++k) {
-    if (threadIdx.x == 0) {
-      int p = k;
+    // the first of the largest, by the lanes of the first wave (rows i, i + 64, ... in turn, then the
+    // smaller row of equal values between lanes)
+    if (threadIdx.x < 64) {
+      int p = m;
       double best = -1;
-      for (int i = k; i < m; ++i) {
+      for (int i = k + threadIdx.x; i < m; i += 64) {
         const double v = fabs(Q[k * m + i].x) + fabs(Q[k * m + i].y);
         if (v > best) { best = v; p = i; }
       }
-      piv_ws[k] = p;
+      for (int off = 32; off > 0; off >>= 1) {
+        const double v = __shfl_xor(best, off, 64);
+        const int q = __shfl_xor(p, off, 64);
+        if (v > best || (v == best && q < p)) { best = v; p = q; }
+      }
+      if (threadIdx.x == 0) piv_ws[k] = p < m ? p : k;  // no value compares (NaN): no interchange
     }
     __syncthreads();
     const int p = piv_ws[k];
@@ -120,11 +130,13 @@ __device__ inline void pade_exp_wg(const double2* __restrict__ Hm, int m, double
     }
     for (int i = 0; i < m; ++i) {
       double2 acc = b[i];
+#pragma unroll 4
       for (int k = 0; k < i; ++k) acc = csub(acc, cmul(Q[k * m + i], b[k]));
       b[i] = acc;
     }
     for (int i = m - 1; i >= 0; --i) {
       double2 acc = b[i];
+#pragma unroll 4
       for (int k = i + 1; k < m; ++k) acc = csub(acc, cmul(Q[k * m + i], b[k]));
       b[i] = cdiv(acc, Q[i * m + i]);
     }
@@ -140,8 +152,9 @@ __device__ inline void pade_exp_wg(const double2* __restrict__ Hm, int m, double
   __syncthreads();
   for (int i = 0; i < s_scale; ++i) {
     matmul(E, E, T);
-    for (int idx = threadIdx.x; idx < mm; idx += blockDim.x) E[idx] = T[idx];
-    __syncthreads();
+    double2* swap = E;
+    E = T;
+    T = swap;
   }
   for (int i = threadIdx.x; i < m; i += blockDim.x) out_col[i] = E[i];  // column 0
   if (threadIdx.x == 0) *err = E[m - 1];
