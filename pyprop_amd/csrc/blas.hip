@@ -50,37 +50,52 @@ __device__ inline double2 block_sum(double2 v, double2* sh) {
   return r;
 }
 
-// partial[b * width + j] for j in [j0, j0 + g): sum over this block's chunk of conj(V_j) w;
-// when include_norm, partial[b * width + m] = sum |w|^2
+// partial[b * width + j] for the kDotGroup products j of group blockIdx.y: sum over this block's chunk
+// of conj(V_j) w; the product after the last (j = m) is sum |w|^2.  A group per workgroup: one workgroup
+// per chunk for all of them walked through the groups with two barriers per product, 15.0 us on
+// average over the 2 .. 20 vectors of 960 elements (one chunk) of a pAMP step; 8.0 now, each sum in the
+// same order.  (With 74 chunks of 151200 elements it is the vectors that are waited for: 14 us both ways.)
 __global__ __launch_bounds__(kRedThreads) void block_dot_kernel(long long n, int m, const double2* __restrict__ V,
                                                                  long long ld, const double2* __restrict__ w,
                                                                  double2* __restrict__ partial, int width,
                                                                  const int* cond) {
   if (cond && *cond == 0) return;
-  __shared__ double2 sh[kRedThreads / 64];
+  __shared__ double2 sh[kDotGroup][kRedThreads / 64];
   const long long chunk = (n + gridDim.x - 1) / gridDim.x;
   const long long beg = chunk * blockIdx.x;
   const long long end = min(n, beg + chunk);
-  for (int j0 = 0; j0 <= m; j0 += kDotGroup) {
-    double2 acc[kDotGroup];
+  const int j0 = blockIdx.y * kDotGroup;
+  double2 acc[kDotGroup];
 #pragma unroll
-    for (int g = 0; g < kDotGroup; ++g) acc[g] = make_double2(0, 0);
-    for (long long i = beg + threadIdx.x; i < end; i += blockDim.x) {
-      const double2 wv = w[i];
-#pragma unroll
-      for (int g = 0; g < kDotGroup; ++g) {
-        const int j = j0 + g;
-        if (j < m) cfmac(acc[g], V[j * ld + i], wv);
-        else if (j == m) { acc[g].x = fma(wv.x, wv.x, acc[g].x); acc[g].x = fma(wv.y, wv.y, acc[g].x); }
-      }
-    }
+  for (int g = 0; g < kDotGroup; ++g) acc[g] = make_double2(0, 0);
+  for (long long i = beg + threadIdx.x; i < end; i += blockDim.x) {
+    const double2 wv = w[i];
 #pragma unroll
     for (int g = 0; g < kDotGroup; ++g) {
       const int j = j0 + g;
-      if (j > m) break;
-      double2 s = block_sum(acc[g], sh);
-      if (threadIdx.x == 0) partial[(long long)blockIdx.x * width + j] = s;
+      if (j < m) cfmac(acc[g], V[j * ld + i], wv);
+      else if (j == m) { acc[g].x = fma(wv.x, wv.x, acc[g].x); acc[g].x = fma(wv.y, wv.y, acc[g].x); }
     }
+  }
+  // wave sums, then the waves in order (block_sum for the group's products at once)
+#pragma unroll
+  for (int g = 0; g < kDotGroup; ++g)
+    for (int off = 32; off > 0; off >>= 1) {
+      acc[g].x += __shfl_down(acc[g].x, off, 64);
+      acc[g].y += __shfl_down(acc[g].y, off, 64);
+    }
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int g = 0; g < kDotGroup; ++g) sh[g][threadIdx.x >> 6] = acc[g];
+  }
+  __syncthreads();
+  if (threadIdx.x < kDotGroup && j0 + (int)threadIdx.x <= m) {
+    double2 r = make_double2(0, 0);
+    for (int k = 0; k < kRedThreads / 64; ++k) {
+      r.x += sh[threadIdx.x][k].x;
+      r.y += sh[threadIdx.x][k].y;
+    }
+    partial[(long long)blockIdx.x * width + j0 + threadIdx.x] = r;
   }
 }
 
@@ -115,7 +130,8 @@ void block_dot_if(long long n, int m, const double2* V, long long ld, const doub
   const int blocks = reduction_blocks(n);
   const int width = m + 1;
   red.ensure(blocks, width);
-  hipLaunchKernelGGL(block_dot_kernel, dim3(blocks), dim3(kRedThreads), 0, s, n, m, V, ld, w, red.partial.ptr, width,
+  hipLaunchKernelGGL(block_dot_kernel, dim3(blocks, width / kDotGroup + (width % kDotGroup != 0)), dim3(kRedThreads), 0, s,
+                     n, m, V, ld, w, red.partial.ptr, width,
                      cond);
   hipLaunchKernelGGL(finish_kernel, dim3(width), dim3(256), 0, s, red.partial.ptr, blocks, width, width, out_dev,
                      cond);
