@@ -103,7 +103,8 @@ int pp_tp_multiply(const pp_tensor_potential* tp, double scaling, const pp_cplx*
  * counterpart: inner solves of the mixed-precision Cayley step). */
 int pp_tp_multiply_f32(const pp_tensor_potential* tp, float scaling, const pp_cplxf* source,
                        pp_cplxf* dest, pp_stream stream);
-/* Bytes of potential data the plan streams per multiply (for roofline accounting). */
+/* Bytes of potential data the plan holds: values that repeat are stored once, so a multiply
+ * can read some of them several times (from the caches). */
 int pp_tp_info(const pp_tensor_potential* tp, int64_t* stream_bytes, int64_t* tuple_count,
                int* is_real, int* inner_kind);
 int pp_tp_destroy(pp_tensor_potential* tp);
@@ -306,8 +307,9 @@ typedef struct pp_precond pp_precond;
  *   s1, s2: host dense (n1, n1), (n2, n2) overlaps; band = half bandwidth of S (k-1).
  *   p_data: host complex (nchan, p1_count, p2_count) angular-diagonal potential with
  *   Simp pair lists pairs1 (p1_count, 2) and pairs2 (p2_count, 2) for the radial ranks.
- * LU without pivoting (the real part of M_c is positive definite); the SuperLU variant
- * of the reference solves the same systems exactly. */
+ * No pivoting (the real part of M_c is positive definite); the SuperLU variant of the
+ * reference solves the same systems exactly.  Real symmetric S and P with n2 <= 64 and
+ * band <= 8 are factorized in superblocks of band block rows, everything else as a block LU. */
 int pp_precond_create(int nchan, int n1, int n2, int band, const double* s1, const double* s2,
                       const pp_cplx* p_data, int p1_count, const int32_t* pairs1, int p2_count,
                       const int32_t* pairs2, pp_cplx scaling_h, pp_cplx scaling_s,
