@@ -268,9 +268,10 @@ __global__ __launch_bounds__(256) void pamp_newvec_kernel(long long n, const dou
   if (blockIdx.x == 0) {
     if (h)
       for (int i = threadIdx.x; i <= j; i += blockDim.x) H[j * m + i] = h[i];
+    __syncthreads();  // every wave has read the flag above and stored its coefficients
     if (threadIdx.x == 0) {
       if (broken) {
-        flags[0] = 1;  // (a block that starts later and sees it does what it would do anyway)
+        flags[0] = 1;  // (another block that sees it leaves, as it would by its own beta)
       } else {
         H[j * m + (j + 1)] = make_double2(beta, 0);
         sc[1] = make_double2(1.0 / beta, 0);
