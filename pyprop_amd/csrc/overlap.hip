@@ -344,7 +344,7 @@ static void overlap_tile(const OverlapFactor& ov, int op, bool conj, long long p
 // would otherwise compute both.
 __device__ inline double divide_by(double x, double c, double r) {
   double q = x * r;
-  const bool plain = (fabs(q) > 1e-250 && fabs(q) < 1e250) || x == 0.0;
+  const bool plain = (fabs(q) > 1e-250 && fabs(q) < 1e250) || (x == 0.0 && q == 0.0);
   q = fma(fma(-q, c, x), r, q);
   q = fma(fma(-q, c, x), r, q);
   if (__ballot(!plain)) q = plain ? q : x / c;

@@ -21,7 +21,7 @@ def torch():
     return t
 
 
-def _overlap(n, sd, seed=0):
+def _overlap(n, sd, seed=0, scale=1.0):
     """A banded positive definite S, its upper band, the device object and its factor U (extended)."""
     from pyprop_amd.propagator import OverlapMatrix
     rng = np.random.default_rng(seed)
@@ -29,6 +29,7 @@ def _overlap(n, sd, seed=0):
     for d in range(1, sd + 1):
         v = rng.uniform(-0.5, 0.5, n - d) / sd
         S += np.diag(v, d) + np.diag(v, -d)
+    S *= scale
     ov = OverlapMatrix(S, sd)
     from pyprop_amd import _native as N, device as D
     band = np.zeros((n, sd + 1))
@@ -122,3 +123,19 @@ def test_overlap_substitution_extreme_values(torch, n, sd):
     assert np.all(_apply(torch, ov, SQRT_SOLVE, False, x) == 0)
     x[0, 0, 0] = np.inf
     assert np.isinf(_apply(torch, ov, SQRT_SOLVE, True, x)[0, 0, 0].real)
+
+
+# factors of 1e-35 and 1e35 lie outside the range whose reciprocals are formed (2^+-100), the others inside
+@pytest.mark.parametrize("scale", [1e-70, 1e-56, 1e56, 1e70])
+@pytest.mark.parametrize("n,sd", [(9, 8), (120, 6), (512, 3)])
+def test_overlap_substitution_of_zeros_with_extreme_factors(torch, n, sd, scale):
+    """Zeros stay zeros and the rest is the quotient, whatever the scale of S."""
+    ov, U = _overlap(n, sd, seed=n, scale=scale)
+    x = np.zeros((3, n, 1), complex)
+    x[1, n // 2] = 1.0 - 0.5j
+    x[2, 0] = 2.0  # the imaginary part is zero throughout
+    for conj in (False, True):
+        got = _apply(torch, ov, SQRT_SOLVE, conj, x)
+        ref = _reference(U, SQRT_SOLVE, conj, x[:, :, 0].T.astype(np.clongdouble)).T
+        assert np.all(got[0] == 0) and np.all(got[2].imag == 0)
+        assert np.max(np.abs(got[:, :, 0] - ref)) < 2.0 ** -53 * 10 * (sd + 16) * np.max(np.abs(ref))
