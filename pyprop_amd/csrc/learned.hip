@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "pp_common.h"
@@ -86,20 +87,25 @@ struct GemmFrag {
   u32x4 v[2];
 };
 
-// Thread t's share of the tile rows r0..r0+63, k0..k0+63 of X(r, k) = p[r*sr + k*sk], zeros outside.
+// How an operand is read (gemm_form): 16 bytes at a time; value by value through range-checked loads
+// too, so that in neither form a load waits at a branch; or value by value from any address.
+enum { kWide = 2, kSingle = 1, kAnyStride = 0 };
+
+// Thread t's share of the tile rows r0..r0+63, k0..k0+63 of X(r, k) = p[r*sr + k*sk], zeros outside
+// (in the range-checked forms by an offset past the range).
 // KC (k contiguous): rows t / 8 and t / 8 + 32, k chunk t % 8.  Otherwise rows 8 (t % 8) .. + 7 at
-// k = 2 (t / 8) and the next.  WIDE (see gemm_wide): 16-byte range-checked loads, a share outside
-// the operand past the range, so that no load waits at a branch.
-template <bool KC, bool WIDE>
+// k = 2 (t / 8) and the next.
+template <bool KC, int FORM>
 __device__ __forceinline__ GemmFrag gemm_load(const uint16_t* __restrict__ p, long long sr, long long sk, int R, int r0,
                                               int k0, int ke, int t) {
   GemmFrag f;
-  const __amdgpu_buffer_rsrc_t tile = rsrc(p + (KC ? (long long)r0 * sr : (long long)r0), kOff16 - 16);
+  const __amdgpu_buffer_rsrc_t tile =
+      rsrc(p + (FORM == kSingle ? r0 * sr + k0 * sk : KC ? (long long)r0 * sr : (long long)r0), kOff16 - 16);
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int r = KC ? r0 + (t >> 3) + 32 * h : r0 + (t & 7) * 8;
     const int k = KC ? k0 + (t & 7) * 8 : k0 + (t >> 3) * 2 + h;
-    if (WIDE) {
+    if (FORM == kWide) {
       const int off = KC ? ((r - r0) * (int)sr + k) * 2 : (k * (int)sk + (r - r0)) * 2;
       f.v[h] = ld16(tile, r < R && k < ke ? off : kOff16);
     } else {
@@ -109,7 +115,13 @@ __device__ __forceinline__ GemmFrag gemm_load(const uint16_t* __restrict__ p, lo
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const int rr = KC ? r : r + 2 * q + e, kk = KC ? k + 2 * q + e : k;
-          if (rr < R && kk < ke) w[e] = p[(long long)rr * sr + (long long)kk * sk];
+          const bool in = rr < R && kk < ke;
+          if (FORM == kSingle) {
+            const int off = ((rr - r0) * (int)sr + (kk - k0) * (int)sk) * 2;
+            w[e] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(tile, in ? off : kOff16, 0, 0);
+          } else if (in) {
+            w[e] = p[(long long)rr * sr + (long long)kk * sk];
+          }
         }
         f.v[h][q] = w[0] | (w[1] << 16);
       }
@@ -118,13 +130,16 @@ __device__ __forceinline__ GemmFrag gemm_load(const uint16_t* __restrict__ p, lo
   return f;
 }
 
-// Whether an operand of R rows (k in [0, K)) can be read 16 bytes at a time: shares of eight lie
-// inside or outside it as a whole and are 16-byte aligned, and a tile's offsets fit the 31 bits of
-// a buffer offset.
-static bool gemm_wide(const uint16_t* p, int R, int K, long long sr, long long sk) {
-  if (reinterpret_cast<uintptr_t>(p) & 15) return false;
-  if (sk == 1) return sr % 8 == 0 && K % 8 == 0 && sr >= 0 && 2 * (GBM * sr + K) < kOff16 - 16;
-  return sr == 1 && sk % 8 == 0 && R % 8 == 0 && sk >= 0 && 2 * (K * sk + GBM) < kOff16 - 16;
+// The form for an operand of R rows (k in [0, K)).  Wide where shares of eight lie inside or outside
+// it as a whole and are 16-byte aligned; the range-checked forms where a tile's offsets fit the 31
+// bits of a buffer offset.
+static int gemm_form(const uint16_t* p, int R, int K, long long sr, long long sk) {
+  if (sr < 0 || sk < 0) return kAnyStride;
+  if ((reinterpret_cast<uintptr_t>(p) & 15) == 0) {
+    if (sk == 1 && sr % 8 == 0 && K % 8 == 0 && 2 * (GBM * sr + K) < kOff16 - 16) return kWide;
+    if (sk != 1 && sr == 1 && sk % 8 == 0 && R % 8 == 0 && 2 * (K * sk + GBM) < kOff16 - 16) return kWide;
+  }
+  return 2 * (GBM * sr + GBK * sk) < kOff16 - 16 ? kSingle : kAnyStride;
 }
 
 template <bool KC>
@@ -147,7 +162,7 @@ __device__ __forceinline__ void gemm_store(const GemmFrag& f, uint16_t* S, int t
   }
 }
 
-template <bool AK, bool BK, bool WIDE>
+template <bool AK, bool BK, int AF, int BF>
 __global__ __launch_bounds__(256) void gemm_bf16_kernel(int M, int N, int K, int kchunk, const uint16_t* __restrict__ a,
                                                         long long sam, long long sak, const uint16_t* __restrict__ b,
                                                         long long sbk, long long sbn, float* __restrict__ c) {
@@ -170,18 +185,18 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(int M, int N, int K, int
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int steps = (ke - kb + GBK - 1) / GBK;
   GemmFrag fa[2], fb[2];
-  fa[0] = gemm_load<AK, WIDE>(a, sam, sak, M, m0, kb, ke, t);
-  fb[0] = gemm_load<BK, WIDE>(b, sbn, sbk, N, n0, kb, ke, t);  // B viewed as (n, k)
-  fa[1] = gemm_load<AK, WIDE>(a, sam, sak, M, m0, kb + GBK, ke, t);
-  fb[1] = gemm_load<BK, WIDE>(b, sbn, sbk, N, n0, kb + GBK, ke, t);
+  fa[0] = gemm_load<AK, AF>(a, sam, sak, M, m0, kb, ke, t);
+  fb[0] = gemm_load<BK, BF>(b, sbn, sbk, N, n0, kb, ke, t);  // B viewed as (n, k)
+  fa[1] = gemm_load<AK, AF>(a, sam, sak, M, m0, kb + GBK, ke, t);
+  fb[1] = gemm_load<BK, BF>(b, sbn, sbk, N, n0, kb + GBK, ke, t);
   auto step = [&](int s, GemmFrag& ra, GemmFrag& rb) {
     // buffer s & 1 was last read in step s - 2; the barrier of step s - 1 lies in between
     gemm_store<AK>(ra, As[s & 1], t);
     gemm_store<BK>(rb, Bs[s & 1], t);
     // past the last step the loads are masked: issued all the same, so that the compiler knows
     // how many are in flight and waits for the older step's only
-    ra = gemm_load<AK, WIDE>(a, sam, sak, M, m0, kb + (s + 2) * GBK, ke, t);
-    rb = gemm_load<BK, WIDE>(b, sbn, sbk, N, n0, kb + (s + 2) * GBK, ke, t);
+    ra = gemm_load<AK, AF>(a, sam, sak, M, m0, kb + (s + 2) * GBK, ke, t);
+    rb = gemm_load<BK, BF>(b, sbn, sbk, N, n0, kb + (s + 2) * GBK, ke, t);
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -229,24 +244,30 @@ int gemm_bf16(int M, int N, int K, const uint16_t* a, long long sam, long long s
   const int kchunk = (int)ceil_div(ceil_div(K, splits), GBK) * GBK;
   const int z = (int)ceil_div(K, kchunk);
   const dim3 grid((N + GBN - 1) / GBN, (M + GBM - 1) / GBM, z);
-  const bool wide = gemm_wide(a, M, K, sam, sak) && gemm_wide(b, N, K, sbn, sbk);
-#define PP_GEMM(AK, BK)                                                                                              \
-  if (wide)                                                                                                          \
-    hipLaunchKernelGGL((gemm_bf16_kernel<AK, BK, true>), grid, dim3(256), 0, s, M, N, K, kchunk, a, sam, sak, b, sbk, \
-                       sbn, c);                                                                                      \
-  else                                                                                                               \
-    hipLaunchKernelGGL((gemm_bf16_kernel<AK, BK, false>), grid, dim3(256), 0, s, M, N, K, kchunk, a, sam, sak, b,     \
-                       sbk, sbn, c)
-  if (sak == 1 && sbk == 1) {
-    PP_GEMM(true, true);
-  } else if (sak == 1) {
-    PP_GEMM(true, false);
-  } else if (sbk == 1) {
-    PP_GEMM(false, true);
-  } else {
-    PP_GEMM(false, false);
-  }
+  // Each operand by its own layout: the training of an odd number of B-splines multiplies matrices of
+  // 2 n^2 columns, which cannot be read 16 bytes at a time, by matrices of the hidden width, which can:
+  // 512 x 6962 x 256, A rows of 256 and B rows of 6962: 18.4 us (39.5 with both value by value behind
+  // branches; 21.5 one K step of 32 at a time); 256 x 512 x 6962, rows of 6962 in both: 178 (448; 652).
+  // Stored with aligned rows (6968): 177.  A training step at 59 B-splines: 184 us (266; 515).
+  auto launch = [&](auto fa, auto fb) {
+#define PP_GEMM(AK, BK)                                                                                           \
+  hipLaunchKernelGGL((gemm_bf16_kernel<AK, BK, fa.value, fb.value>), grid, dim3(256), 0, s, M, N, K, kchunk, a, sam, \
+                     sak, b, sbk, sbn, c)
+    if (sak == 1 && sbk == 1) PP_GEMM(true, true);
+    else if (sak == 1) PP_GEMM(true, false);
+    else if (sbk == 1) PP_GEMM(false, true);
+    else PP_GEMM(false, false);
 #undef PP_GEMM
+  };
+  const int form_a = gemm_form(a, M, K, sam, sak), form_b = gemm_form(b, N, K, sbn, sbk);
+  constexpr std::integral_constant<int, kWide> wide;
+  constexpr std::integral_constant<int, kSingle> single;
+  constexpr std::integral_constant<int, kAnyStride> any;
+  if (form_a == kAnyStride || form_b == kAnyStride) launch(any, any);
+  else if (form_a == kWide && form_b == kWide) launch(wide, wide);
+  else if (form_a == kWide) launch(wide, single);
+  else if (form_b == kWide) launch(single, wide);
+  else launch(single, single);
   PP_HIP(hipGetLastError());
   return z;
 }

@@ -70,25 +70,31 @@ def test_gradients_at_tile_edges(torch, dims):
         assert np.all(g["emb"][c] == 0)
 
 
-def _bf16_bits(a):
-    return (mlp.bf16(a).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
-
-
 # around the 64 x 64 x 64 tile: below it, exact, one over, K steps 1 to 5 (two are loaded ahead),
-# extents that forbid 16-byte loads
+# extents that forbid 16-byte loads in both operands, in one of them or in none; strides padded to a
+# multiple of eight, so that rows are aligned but their last share is not whole
+@pytest.mark.parametrize("pad", [False, True])
 @pytest.mark.parametrize("a_k", [True, False])
 @pytest.mark.parametrize("b_k", [True, False])
-@pytest.mark.parametrize("dims", [(1, 1, 1), (64, 64, 64), (65, 63, 129), (128, 72, 192), (40, 200, 264), (66, 130, 320)],
+@pytest.mark.parametrize("dims", [(1, 1, 1), (64, 64, 64), (65, 63, 129), (128, 72, 192), (40, 200, 264), (66, 130, 320),
+                                  (64, 66, 40), (130, 72, 100)],
                          ids=lambda d: "x".join(map(str, d)))
-def test_gemm_at_tile_edges(torch, dims, a_k, b_k):
+def test_gemm_at_tile_edges(torch, dims, a_k, b_k, pad):
     from pyprop_amd import _native as N, device as D
     M, N_, K = dims
     rng = np.random.default_rng(M * K)
     A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N_)).astype(np.float32)
-    sam, sak = (K, 1) if a_k else (1, M)
-    sbk, sbn = (1, K) if b_k else (N_, 1)
-    da = torch.from_numpy(_bf16_bits(A if a_k else A.T.copy()).view(np.int16).copy()).to("cuda")
-    db = torch.from_numpy(_bf16_bits(B.T.copy() if b_k else B).view(np.int16).copy()).to("cuda")
+
+    def operand(X):  # rows of X contiguous; the padding holds NaN, which no product may see
+        ld = -(-X.shape[1] // 8) * 8 if pad else X.shape[1]
+        wide = np.full((X.shape[0], ld), np.nan, np.float32)
+        wide[:, :X.shape[1]] = mlp.bf16(X)
+        return torch.from_numpy(wide).to("cuda").to(torch.bfloat16), ld
+
+    da, lda = operand(A if a_k else A.T)
+    db, ldb = operand(B.T if b_k else B)
+    sam, sak = (lda, 1) if a_k else (1, lda)
+    sbk, sbn = (1, ldb) if b_k else (ldb, 1)
     dc = torch.full((M + 1, N_), 7.0, dtype=torch.float32, device="cuda")
     N.check(N.load().pp_gemm_bf16(M, N_, K, D.ptr(da), sam, sak, D.ptr(db), sbk, sbn, D.ptr(dc), D.stream_handle()))
     got = dc.cpu().numpy().astype(np.float64)
@@ -96,6 +102,20 @@ def test_gemm_at_tile_edges(torch, dims, a_k, b_k):
     # exact products of BF16 values, K FP32 additions
     bound = K * 2.0 ** -24 * (np.abs(mlp.bf16(A)) @ np.abs(mlp.bf16(B)))
     assert np.all(np.abs(got[:M] - mlp.bf16(A) @ mlp.bf16(B)) <= bound + 1e-30)
+
+
+def test_gemm_of_any_strides(torch):
+    """A with its rows in descending order, B with every other column: read value by value."""
+    from pyprop_amd import _native as N, device as D
+    rng = np.random.default_rng(0)
+    M, N_, K = 70, 66, 72
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, 2 * N_)).astype(np.float32)
+    da, db = (torch.from_numpy(x).to("cuda").to(torch.bfloat16) for x in (A, B))
+    dc = torch.empty((M, N_), dtype=torch.float32, device="cuda")
+    N.check(N.load().pp_gemm_bf16(M, N_, K, da[M - 1].data_ptr(), -K, 1, D.ptr(db), 2 * N_, 2, D.ptr(dc),
+                                  D.stream_handle()))
+    a, b = mlp.bf16(A)[::-1], mlp.bf16(B)[:, ::2]
+    assert np.all(np.abs(dc.cpu().numpy() - a @ b) <= K * 2.0 ** -24 * (np.abs(a) @ np.abs(b)))
 
 
 # parameter counts with and without a remainder of two past the 16-byte groups, hidden widths whose
