@@ -339,12 +339,12 @@ static void overlap_tile(const OverlapFactor& ov, int op, bool conj, long long p
 
 // x / c for r = 1 / c rounded: two residual corrections of x r give the rounded quotient (P. Markstein,
 // IBM J. Res. Dev. 34 (1990) 111), the bits of the division (0 for x = -0), in five dependent
-// operations instead of its ten.  Where a residual could underflow or a value is not finite (r NaN:
-// a divisor outside 2^+-100) the division itself, behind a branch of the whole wave: the compiler
-// would otherwise compute both.
+// operations instead of its ten.  Where a residual could underflow or a value is not finite, and for
+// r = 0 (a divisor outside 2^+-100), the division itself, behind a branch of the whole wave: the
+// compiler would otherwise compute both.
 __device__ inline double divide_by(double x, double c, double r) {
   double q = x * r;
-  const bool plain = (fabs(q) > 1e-250 && fabs(q) < 1e250) || (x == 0.0 && q == 0.0);
+  const bool plain = (fabs(q) > 1e-250 && fabs(q) < 1e250) || x == 0.0;
   q = fma(fma(-q, c, x), r, q);
   q = fma(fma(-q, c, x), r, q);
   if (__ballot(!plain)) q = plain ? q : x / c;
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(256) void overlap_chain_kernel(const double* __rest
     } else {
       const double c = r < n ? u[i * (SD + 1) + SD] : 1.0;
       C[r * W + SD] = c;
-      C[r * W + SD + 1] = c > 0x1p-100 && c < 0x1p100 ? 1.0 / c : __builtin_nan("");
+      C[r * W + SD + 1] = c > 0x1p-100 && c < 0x1p100 ? 1.0 / c : 0.0;
     }
   }
   __syncthreads();
