@@ -6,11 +6,11 @@
 // applied to every 1-D fibre of one rank of a C-ordered tensor (MapToRank3 loops,
 // :155-229).
 //
-// Up to kTileRows rows a workgroup holds a tile of whole fibres in LDS: the multiplies are banded
-// sums out of LDS and S^-1 x is a product with the dense inverse, which the host forms in extended
-// precision (overlap_tile_kernel); U^-1 x and U^-H x are substitutions by one lane per fibre with
-// the rows and coefficients staged (overlap_chain_kernel).  Beyond, one thread owns one fibre
-// (substitution) or one element (multiply).
+// Up to kTileRows rows and not too many fibres (in_tiles) a workgroup holds a tile of whole fibres in
+// LDS: the multiplies are banded sums out of LDS and S^-1 x is a product with the dense inverse, which
+// the host forms in extended precision (overlap_tile_kernel); U^-1 x and U^-H x are substitutions by
+// one lane per fibre with the rows and coefficients staged (overlap_chain_kernel).  Beyond, one thread
+// owns one fibre (substitution) or one element (multiply).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -196,13 +196,17 @@ struct FibreTile {
   long long base, row, fibre;
   int cnt;
 };
+// Workgroup b runs on XCD b % 8: each XCD takes a contiguous range of tiles, so that a cache line that
+// two tiles share comes into one L2.
 template <int FT>
 __device__ inline FibreTile fibre_tile(int n, long long pre, long long post) {
+  const unsigned id = blockIdx.x, per_xcd = gridDim.x >> 3;
+  const long long tile = (id & 7) * per_xcd + min(id & 7, gridDim.x & 7) + (id >> 3);
   if (post > 1) {
-    const long long tiles = (post + FT - 1) / FT, p = blockIdx.x / tiles, q0 = (blockIdx.x - p * tiles) * FT;
+    const long long tiles = (post + FT - 1) / FT, p = tile / tiles, q0 = (tile - p * tiles) * FT;
     return {p * n * post + q0, post, 1, (int)min((long long)FT, post - q0)};
   }
-  const long long p0 = blockIdx.x * (long long)FT;
+  const long long p0 = tile * FT;
   return {p0 * n, 1, n, (int)min((long long)FT, pre - p0)};
 }
 // element e of the tile in memory order: consecutive threads on consecutive addresses
@@ -233,7 +237,8 @@ static long long tile_count(long long pre, long long post, int ft) {
 // 64 g .. 64 g + 63 over the k-th part of j for all FT fibres, and the parts are added in order.
 // dst may be src: a workgroup has read its tile before it writes it.  Two substitutions are a chain
 // of 2 n dependent rows with one lane per fibre, 50.5 us per rank at 42 x 60 x 60; the product has
-// none, 10.9 us.  The two banded passes of U^H U in one launch: 2 x 5.0 us -> 5.6.
+// none, 10.9 us.  The two banded passes of U^H U in one launch: 2 x 5.0 us -> 5.6 (42 x 512 x 60: 31 us
+// -> 25, 72 with one fibre per workgroup and consecutive tiles on different XCDs).
 template <int FT>
 __global__ __launch_bounds__(1024) void overlap_tile_kernel(const double* __restrict__ u,
                                                             const double* __restrict__ Sinv, int mul_first,
@@ -245,7 +250,7 @@ __global__ __launch_bounds__(1024) void overlap_tile_kernel(const double* __rest
   const FibreTile t = fibre_tile<FT>(n, pre, post);
   load_tile<FT>(t, n, src, X);
   if (!Sinv) {
-    double* C = reinterpret_cast<double*>(tile + 2 * n * FT);
+    double* C = reinterpret_cast<double*>(tile + (mul_second >= 0 ? 2 : 1) * n * FT);
     for (int e = threadIdx.x; e < n * (sd + 1); e += blockDim.x) C[e] = u[e];
     __syncthreads();
     auto band = [&](const double2* in, int mode, int i, int f) {
@@ -311,6 +316,11 @@ __global__ __launch_bounds__(1024) void overlap_tile_kernel(const double* __rest
   }
 }
 
+// coefficients of sd superdiagonals (-1: none)
+static size_t tile_lds(int n, int ft, int parts, int sd) {
+  return (size_t)n * ft * (1 + parts) * sizeof(double2) + (size_t)n * (sd + 1) * sizeof(double);
+}
+
 static void overlap_tile(const OverlapFactor& ov, int op, bool conj, long long pre, long long post, const double2* src,
                          double2* dst, hipStream_t s) {
   const int n = ov.n, groups = (n + 63) / 64;
@@ -318,11 +328,14 @@ static void overlap_tile(const OverlapFactor& ov, int op, bool conj, long long p
   const bool solve = op == PP_OVERLAP_SOLVE;
   const int first = op == PP_OVERLAP_MULTIPLY ? 0 : conj ? 1 : 0, second = op == PP_OVERLAP_MULTIPLY ? 1 : -1;
   // few fibres: one per workgroup, so that as many CUs as there are take part; many: tiles whose
-  // coefficients are read once for FT fibres, as wide as leaves 64 KB of LDS for the partial sums
-  const int ft = fibres <= 512 ? 1 : n <= 64 ? (solve ? 8 : 4) : n <= 160 ? 4 : n <= 320 ? 2 : 1;
-  const int parts = solve ? std::max(1, std::min(ft >= 4 ? 4 : 8, 16 / groups)) : 1;
-  const int threads = solve ? 64 * groups * parts : 256;
-  const size_t lds = (size_t)n * ft * (1 + parts) * sizeof(double2) + (solve ? 0 : (size_t)n * (ov.sd + 1) * sizeof(double));
+  // coefficients are read once for FT fibres.  A solve's are as wide as leaves 64 KB of LDS for the
+  // partial sums; a multiply's have four fibres, as narrower ones of a rank that is not the last take
+  // less than 64 bytes of a row and a cache line then goes to several XCDs
+  const bool few = fibres <= (solve || post == 1 ? 512 : 128);
+  const int ft = few ? 1 : post == 2 ? 2 : solve && n <= 64 ? 8 : n <= 160 || (!solve && post > 1) ? 4 : n <= 320 ? 2 : 1;
+  const int parts = solve ? std::max(1, std::min(ft >= 4 ? 4 : 8, 16 / groups)) : second < 0 ? 0 : 1;
+  const int threads = solve ? 64 * groups * parts : n * ft <= 640 ? 256 : 1024;
+  const size_t lds = tile_lds(n, ft, parts, solve ? -1 : ov.sd);
   const long long blocks = tile_count(pre, post, ft);
   PP_REQUIRE(blocks <= 0x7fffffffLL, "too many fibres");
 #define PP_TILE(F)                                                                                             \
@@ -435,8 +448,8 @@ template <int SD>
 static void overlap_chain(const OverlapFactor& ov, bool lower, long long pre, long long post, const double2* src,
                           double2* dst, hipStream_t s) {
   // few fibres: two per workgroup (the chain costs the same for any number; the copies shrink);
-  // many: 16, as long as the tile leaves a CU several workgroups
-  const int n = ov.n, ft = pre * post <= 512 || n > 160 ? 2 : 16;
+  // many: 16, as long as the tile leaves a CU several workgroups (or, if only two of them are filled, all)
+  const int n = ov.n, ft = pre * post <= 512 || (post == 2 && n > 128) || n > 160 ? 2 : 16;
   const int rows = (n + SD - 1) / SD * SD;
   const size_t lds = (size_t)(rows + 2) * (ft * sizeof(double2) + (SD + 2) * sizeof(double));
   const long long blocks = tile_count(pre, post, ft);
@@ -491,6 +504,33 @@ static void launch_window(int op, bool conj, const double* u, int n, long long p
 #undef PP_OW
 }
 
+// Whether an operation runs on tiles of fibres in LDS; otherwise a thread takes a fibre or an element.
+// A substitution by threads is a chain of n rows that takes the same time for any number of fibres
+// until they fill the chip; on tiles it is several times shorter, but a workgroup has few chains (or
+// multiplies by n^2 values), so its time grows with the fibres.  us by threads / on tiles, six
+// superdiagonals:
+//   fibres x rows   2520 x 60  20000 x 60  80000 x 60  20000 x 160  2520 x 200  20000 x 200  2520 x 512
+//   S^-1              46 / 9     48 / 29     91 / 101    137 / 132    150 / 35    175 / 241    406 / 311
+//     (two superdiagonals, 20000 x 160: 108 / 131)
+//   U^-1              35 / 11    36 / 15     51 / 45     110 / 57     114 / 45    139 / 181    287 / 134
+//   U^-H              22 / 11    21 / 15     48 / 45      61 / 58      69 / 45     78 / 180    173 / 135
+// and 20000 x 512 up to five times slower on tiles.  Below 16 rows both take the launch.
+// The multiplies have no chain, and spare a pass over memory on tiles.
+static bool in_tiles(const OverlapFactor& ov, int op, bool conj, long long fibres) {
+  const int n = ov.n;
+  if (n > kTileRows) return false;
+  const long long values = fibres * n;
+  if (op == PP_OVERLAP_SOLVE)
+    return n >= 16 && fibres <= 32768 && values <= (n <= 160 && ov.sd >= 6 ? 3200000 : n <= 320 ? 2500000 : 1300000);
+  if (op == PP_OVERLAP_SQRT_SOLVE) {
+    if (ov.sd < 1 || ov.sd > 8 || n < 16) return false;
+    if (n <= 160) return fibres <= 32768 && (!conj || values <= 3200000);
+    const long long work = values * (std::max(ov.sd, 6) + 2);
+    return conj ? fibres <= 4000 && work <= 8 * 1300000 : work <= 8 * 2600000;
+  }
+  return ov.sd <= 8;
+}
+
 void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const int* extents, int rank,
                    const double2* src, double2* data, hipStream_t s, double2* work) {
   PP_REQUIRE(rank >= 0 && rank < ndim, "rank out of range");
@@ -503,12 +543,11 @@ void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const i
   const int blocks = ceil_div(fibres, threads);
   if (blocks == 0) return;
   PP_REQUIRE(op >= 0 && op <= 3, "unknown overlap op");
-  // (512 rows of 8 superdiagonals: 53 KB of LDS with the multiply's coefficients)
-  if (ov.n <= kTileRows && (op == PP_OVERLAP_SOLVE || (op != PP_OVERLAP_SQRT_SOLVE && ov.sd <= 8))) {
-    overlap_tile(ov, op, conj, pre, post, src, data, s);
-    return;
-  }
-  if (ov.n <= kTileRows && ov.sd >= 1 && ov.sd <= 8) {
+  if (in_tiles(ov, op, conj, fibres)) {
+    if (op != PP_OVERLAP_SQRT_SOLVE) {
+      overlap_tile(ov, op, conj, pre, post, src, data, s);
+      return;
+    }
     switch (ov.sd) {
 #define PP_CH(K) case K: overlap_chain<K>(ov, conj, pre, post, src, data, s); break;
       PP_CH(1) PP_CH(2) PP_CH(3) PP_CH(4) PP_CH(5) PP_CH(6) PP_CH(7) PP_CH(8)
@@ -516,7 +555,6 @@ void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const i
     }
     return;
   }
-  if (src != data) vec_copy(fibres * ov.n, src, data, s);
   if (ov.sd >= 1 && ov.sd <= 8 && (op == PP_OVERLAP_MULTIPLY || op == PP_OVERLAP_SQRT_MULTIPLY)) {
     const long long total = pre * ov.n * post;
     if (!work && ov.work.count < (size_t)total) ov.work.resize(total);
@@ -532,8 +570,10 @@ void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const i
       }
     };
     if (op == PP_OVERLAP_MULTIPLY) {
-      pass(0, data, w);     // U x
+      pass(0, src, w);      // U x
       pass(1, w, data);     // U^H (U x)
+    } else if (src != data) {
+      pass(conj ? 1 : 0, src, data);
     } else {
       pass(conj ? 1 : 0, data, w);
       PP_HIP(hipMemcpyAsync(data, w, total * sizeof(double2), hipMemcpyDeviceToDevice, s));
@@ -541,6 +581,7 @@ void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const i
     PP_HIP(hipGetLastError());
     return;
   }
+  if (src != data) vec_copy(fibres * ov.n, src, data, s);
   if (ov.sd >= 1 && ov.sd <= 8) {
     switch (ov.sd) {
 #define PP_SD(K) case K: launch_window<K>(op, conj, ov.u.ptr, ov.n, pre, post, data, blocks, threads, s); break;
@@ -602,7 +643,12 @@ extern "C" int pp_overlap_create(int n, int superdiagonals, const double* s_uppe
       o->f.sd = superdiagonals;
       band_cholesky_upper_host(n, superdiagonals, s_upper, o->f.u_host);
       o->f.u.upload(o->f.u_host.data(), o->f.u_host.size());
-      if (n <= kTileRows) invert_overlap(o->f);
+      if (n <= kTileRows) {
+        invert_overlap(o->f);
+        // 102 KB at 512 rows of 8 superdiagonals
+        PP_HIP(hipFuncSetAttribute((const void*)overlap_tile_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)tile_lds(kTileRows, 4, 1, 8)));
+      }
       PP_HIP(hipDeviceSynchronize());
     } catch (...) {
       delete o;

@@ -116,8 +116,9 @@ struct OverlapFactor {
   DeviceBuffer<double> s_inv;    // S^-1, dense, up to the tile kernel's rows
   mutable DeviceBuffer<double2> work;  // out-of-place passes of the multiply ops (grown on demand)
 };
-// data <- op src along one rank (src may be data).  Beyond the tile kernel's rows the multiply ops
-// need an out-of-place buffer: work (as many elements as data); NULL uses ov.work, grown on demand
+// data <- op src along one rank (src may be data).  Where they do not run on tiles (more than 512 rows
+// or 8 superdiagonals) the multiply ops need an out-of-place buffer: work (as many elements as data);
+// NULL uses ov.work, grown on demand
 void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const int* extents, int rank,
                    const double2* src, double2* data, hipStream_t s, double2* work = nullptr);
 

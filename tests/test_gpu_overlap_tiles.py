@@ -1,6 +1,6 @@
 """GPU tests of the overlap operations along one rank at the edges of the tile kernel: row counts
-around a wave and around each tile width, the last size with dense inverse factors and the first
-without, few and many fibres, first, middle and last ranks, against the factor in extended
+around a wave and around each tile width, the last size with a dense inverse and the first without, few
+and many fibres, first, middle and last ranks, against the factor in extended
 precision."""
 import ctypes as C
 
@@ -41,28 +41,37 @@ def _overlap(n, sd, seed=0, scale=1.0):
     return ov, U
 
 
+_BAND = 12  # more than any test's superdiagonals: the entries beyond are zero
+
+
 def _solve_upper(U, b):
     x = b.copy()
     for i in range(U.shape[0] - 1, -1, -1):
-        x[i] = (x[i] - U[i, i + 1:] @ x[i + 1:]) / U[i, i]
+        j = slice(i + 1, i + _BAND)
+        x[i] = (x[i] - U[i, j] @ x[j]) / U[i, i]
     return x
 
 
 def _solve_lower(L, b):
     x = b.copy()
     for i in range(L.shape[0]):
-        x[i] = (x[i] - L[i, :i] @ x[:i]) / L[i, i]
+        j = slice(max(0, i - _BAND), i)
+        x[i] = (x[i] - L[i, j] @ x[j]) / L[i, i]
     return x
+
+
+def _multiply(U, b):
+    return np.stack([U[i, max(0, i - _BAND):i + _BAND] @ b[max(0, i - _BAND):i + _BAND] for i in range(U.shape[0])])
 
 
 def _reference(U, op, conj, x):
     """op applied to the columns of x (extended precision)."""
     if op == MULTIPLY:
-        return U.T @ (U @ x)
+        return _multiply(U.T, _multiply(U, x))
     if op == SOLVE:
         return _solve_upper(U, _solve_lower(U.T, x))
     if op == SQRT_MULTIPLY:
-        return (U.T if conj else U) @ x
+        return _multiply(U.T if conj else U, x)
     return _solve_lower(U.T, x) if conj else _solve_upper(U, x)
 
 
@@ -81,6 +90,20 @@ def _apply(torch, ov, op, conj, x):
 def test_overlap_ops(torch, n, sd, layout):
     if n > 300 and layout[0] * layout[1] > 200:
         layout = (layout[0] % 7 + 1, layout[1] % 7 + 1)
+    _check_ops(torch, n, sd, layout)
+
+
+# more than 64 KB of LDS per multiply; pairs of fibres; fibre counts on both sides of the lines from
+# which on a thread takes a fibre of a substitution
+@pytest.mark.parametrize("n,sd,layout", [(512, 8, (3, 50)), (321, 3, (2, 131)), (160, 6, (300, 2)), (400, 5, (260, 2)),
+                                         (15, 6, (600, 1)), (16, 6, (600, 1)), (17, 4, (32768, 1)), (17, 4, (32769, 1)),
+                                         (321, 2, (5, 810)), (161, 1, (1, 4000)), (161, 1, (4001, 1)),
+                                         (505, 3, (2, 1290))], ids=str)
+def test_overlap_ops_at_the_lines_between_forms(torch, n, sd, layout):
+    _check_ops(torch, n, sd, layout)
+
+
+def _check_ops(torch, n, sd, layout):
     ov, U = _overlap(n, sd, seed=n)
     pre, post = layout
     rng = np.random.default_rng(pre + post)
