@@ -321,7 +321,11 @@ static size_t tile_lds(int n, int ft, int parts, int sd) {
   return (size_t)n * ft * (1 + parts) * sizeof(double2) + (size_t)n * (sd + 1) * sizeof(double);
 }
 
-static void overlap_tile(const OverlapFactor& ov, int op, bool conj, long long pre, long long post, const double2* src,
+// A launch holds fewer than 2^32 threads.
+static bool launchable(long long blocks, int threads) { return blocks * threads < (1LL << 32); }
+
+// false: more tiles than a launch can hold, nothing was done
+static bool overlap_tile(const OverlapFactor& ov, int op, bool conj, long long pre, long long post, const double2* src,
                          double2* dst, hipStream_t s) {
   const int n = ov.n, groups = (n + 63) / 64;
   const long long fibres = pre * post;
@@ -337,7 +341,7 @@ static void overlap_tile(const OverlapFactor& ov, int op, bool conj, long long p
   const int threads = solve ? 64 * groups * parts : n * ft <= 640 ? 256 : 1024;
   const size_t lds = tile_lds(n, ft, parts, solve ? -1 : ov.sd);
   const long long blocks = tile_count(pre, post, ft);
-  PP_REQUIRE(blocks <= 0x7fffffffLL, "too many fibres");
+  if (!launchable(blocks, threads)) return false;
 #define PP_TILE(F)                                                                                             \
   case F:                                                                                                      \
     hipLaunchKernelGGL(overlap_tile_kernel<F>, dim3((unsigned)blocks), dim3(threads), lds, s, ov.u.ptr,        \
@@ -348,6 +352,7 @@ static void overlap_tile(const OverlapFactor& ov, int op, bool conj, long long p
   }
 #undef PP_TILE
   PP_HIP(hipGetLastError());
+  return true;
 }
 
 // x / c for r = 1 / c rounded: two residual corrections of x r give the rounded quotient (P. Markstein,
@@ -452,8 +457,7 @@ static void overlap_chain(const OverlapFactor& ov, bool lower, long long pre, lo
   const int n = ov.n, ft = pre * post <= 512 || (post == 2 && n > 128) || n > 160 ? 2 : 16;
   const int rows = (n + SD - 1) / SD * SD;
   const size_t lds = (size_t)(rows + 2) * (ft * sizeof(double2) + (SD + 2) * sizeof(double));
-  const long long blocks = tile_count(pre, post, ft);
-  PP_REQUIRE(blocks <= 0x7fffffffLL, "too many fibres");
+  const long long blocks = tile_count(pre, post, ft);  // (of at most 32768 fibres: in_tiles)
 #define PP_CHAIN(F, L)                                                                                             \
   hipLaunchKernelGGL((overlap_chain_kernel<SD, F, L>), dim3((unsigned)blocks), dim3(256), lds, s, ov.u.ptr, n, rows, \
                      pre, post, src, dst)
@@ -544,16 +548,13 @@ void overlap_apply(const OverlapFactor& ov, int op, bool conj, int ndim, const i
   if (blocks == 0) return;
   PP_REQUIRE(op >= 0 && op <= 3, "unknown overlap op");
   if (in_tiles(ov, op, conj, fibres)) {
-    if (op != PP_OVERLAP_SQRT_SOLVE) {
-      overlap_tile(ov, op, conj, pre, post, src, data, s);
-      return;
-    }
-    switch (ov.sd) {
-#define PP_CH(K) case K: overlap_chain<K>(ov, conj, pre, post, src, data, s); break;
+    switch (op == PP_OVERLAP_SQRT_SOLVE ? ov.sd : 0) {
+#define PP_CH(K) case K: overlap_chain<K>(ov, conj, pre, post, src, data, s); return;
       PP_CH(1) PP_CH(2) PP_CH(3) PP_CH(4) PP_CH(5) PP_CH(6) PP_CH(7) PP_CH(8)
 #undef PP_CH
+      default:
+        if (overlap_tile(ov, op, conj, pre, post, src, data, s)) return;
     }
-    return;
   }
   if (ov.sd >= 1 && ov.sd <= 8 && (op == PP_OVERLAP_MULTIPLY || op == PP_OVERLAP_SQRT_MULTIPLY)) {
     const long long total = pre * ov.n * post;

@@ -118,6 +118,23 @@ def _check_ops(torch, n, sd, layout):
             assert err < 2.0 ** -53 * 10 * (sd + 16), (op, conj, float(err))
 
 
+def test_more_tiles_than_a_launch_holds(torch):
+    """2^26 + 4 fibres of two rows: at four fibres to a workgroup of 256 threads, over 2^32 threads."""
+    from pyprop_amd import _native as N, device as D
+    fibres = 2 ** 26 + 4
+    if torch.cuda.mem_get_info()[0] < 6 * 32 * fibres:
+        pytest.skip("needs %d GB of device memory" % (6 * 32 * fibres >> 30))
+    ov, U = _overlap(2, 1, seed=2)
+    u00, u01, u11 = (float(U[i, j]) for i, j in ((0, 0), (0, 1), (1, 1)))
+    x = torch.arange(2 * fibres, dtype=torch.float64, device="cuda").remainder_(8191.0).to(torch.complex128)
+    x = x.reshape(fibres, 2)
+    want0, want1 = u00 * x[:, 0] + u01 * x[:, 1], u11 * x[:, 1]
+    ext = np.array([fibres, 2], dtype=np.int32)
+    N.check(N.load().pp_overlap_apply(ov.h, SQRT_MULTIPLY, 0, 2, D.hptr(ext), 1, D.ptr(x), D.stream_handle()))
+    # two products and a sum of values below 2^13
+    assert (x[:, 0] - want0).abs().max().item() < 2.0 ** -38 and (x[:, 1] - want1).abs().max().item() < 2.0 ** -38
+
+
 @pytest.mark.parametrize("n", [64, 100])
 def test_overlap_solve_keeps_nan_where_substitution_does(torch, n):
     """Back substitution carries a NaN of row j to the rows before it, forward to those after."""
