@@ -453,11 +453,11 @@ __global__ void max_abs_imag_kernel(const double2* __restrict__ v, long long n, 
 // (non-temporal).  One value per thread with an integer division and 2 T loads each: 3.45 ms on helium's
 // 1/r12 (394 x 575640, 11 terms, 3.63 GB); this form 0.70 ms (5.2 TB/s; with temporal stores 0.75).
 template <int T>
-__global__ __launch_bounds__(256) void expand_terms_kernel(long long p0, long long rc, long long a_range,
+__global__ __launch_bounds__(256) void expand_terms_kernel(long long p0, long long rc, long long r0, long long a_range,
                                                            const double* __restrict__ coeffs,
                                                            const double* __restrict__ radial,
                                                            double2* __restrict__ out, int accumulate) {
-  const long long r = blockIdx.x * 256LL + threadIdx.x;
+  const long long r = r0 + blockIdx.x * 256LL + threadIdx.x;
   const long long a0 = blockIdx.y * a_range, a1 = min(p0, a0 + a_range);
   if (r >= rc) return;
   double R[T];
@@ -477,22 +477,24 @@ __global__ __launch_bounds__(256) void expand_terms_kernel(long long p0, long lo
 
 void expand_terms(int terms, long long p0, long long rc, const double* coeffs, const double* radial, double2* out,
                   int accumulate, hipStream_t s) {
-  const long long nx = (rc + 255) / 256;
-  PP_REQUIRE(nx <= 0x7fffffffLL, "too many radial values");
-  // a range per workgroup: 4096 workgroups keep every CU writing; more would re-read the radial values
-  const long long ny = std::max(1LL, std::min({p0, 65535LL, (4096 + nx - 1) / nx}));
-  const long long a_range = (p0 + ny - 1) / ny;
-  const dim3 grid((unsigned)nx, (unsigned)((p0 + a_range - 1) / a_range));
-  for (int t0 = 0; t0 < terms; t0 += 12) {
-    switch (std::min(12, terms - t0)) {
-#define PP_EXPAND(T)                                                                                          \
-  case T:                                                                                                     \
-    hipLaunchKernelGGL(expand_terms_kernel<T>, grid, dim3(256), 0, s, p0, rc, a_range, coeffs + t0 * p0,       \
-                       radial + t0 * rc, out, accumulate || t0 > 0);                                          \
+  constexpr long long kSlice = 1LL << 31;  // radial values per launch, which holds fewer than 2^32 threads a row
+  for (long long r0 = 0; r0 < rc; r0 += kSlice) {
+    const long long nx = (std::min(kSlice, rc - r0) + 255) / 256;
+    // a range per workgroup: 4096 workgroups keep every CU writing; more would re-read the radial values
+    const long long ny = std::max(1LL, std::min({p0, 65535LL, (4096 + nx - 1) / nx}));
+    const long long a_range = (p0 + ny - 1) / ny;
+    const dim3 grid((unsigned)nx, (unsigned)((p0 + a_range - 1) / a_range));
+    for (int t0 = 0; t0 < terms; t0 += 12) {
+      switch (std::min(12, terms - t0)) {
+#define PP_EXPAND(T)                                                                                            \
+  case T:                                                                                                       \
+    hipLaunchKernelGGL(expand_terms_kernel<T>, grid, dim3(256), 0, s, p0, rc, r0, a_range, coeffs + t0 * p0,     \
+                       radial + t0 * rc, out, accumulate || t0 > 0);                                            \
     break;
-      PP_EXPAND(1) PP_EXPAND(2) PP_EXPAND(3) PP_EXPAND(4) PP_EXPAND(5) PP_EXPAND(6) PP_EXPAND(7) PP_EXPAND(8)
-      PP_EXPAND(9) PP_EXPAND(10) PP_EXPAND(11) PP_EXPAND(12)
+        PP_EXPAND(1) PP_EXPAND(2) PP_EXPAND(3) PP_EXPAND(4) PP_EXPAND(5) PP_EXPAND(6) PP_EXPAND(7) PP_EXPAND(8)
+        PP_EXPAND(9) PP_EXPAND(10) PP_EXPAND(11) PP_EXPAND(12)
 #undef PP_EXPAND
+      }
     }
   }
   PP_HIP(hipGetLastError());

@@ -34,6 +34,23 @@ def test_expand_potential(torch, dims):
     assert np.all(np.abs(got[:p0].real - c.T @ r) <= 2 * bound)
 
 
+def test_expand_more_radial_values_than_a_launch_holds(torch):
+    """2^32 + 300 radial values, a thread each: two launches."""
+    from pyprop_amd import _native as N, device as D
+    rc, slab = 2 ** 32 + 300, 2 ** 28
+    if torch.cuda.mem_get_info()[0] < 30 * rc:
+        pytest.skip("needs %d GB of device memory" % (30 * rc >> 30))
+    radial = torch.empty(rc, dtype=torch.float64, device="cuda")
+    for a in range(0, rc, slab):
+        radial[a:a + slab] = torch.arange(a, min(rc, a + slab), dtype=torch.float64, device="cuda")
+    coeffs = torch.full((1, 1), 0.5, dtype=torch.float64, device="cuda")
+    out = torch.empty(rc, dtype=torch.complex128, device="cuda")
+    N.check(N.load().pp_expand_potential(1, 1, rc, D.ptr(coeffs), D.ptr(radial), D.ptr(out), D.stream_handle()))
+    for a in range(0, rc, slab):
+        part = out[a:a + slab]
+        assert torch.equal(part.real, 0.5 * radial[a:a + slab]) and not part.imag.any()
+
+
 @pytest.mark.parametrize("kind", ["multipole", "separable"])
 @pytest.mark.parametrize("pairs", [1, 2, 5, 6, 7, 40])  # two terms need six pairs (P1 < 2 Q1) to be combined
 @pytest.mark.parametrize("accumulate", [False, True])
