@@ -34,7 +34,9 @@
 #include <array>
 #include <cstring>
 #include <numeric>
+#include <type_traits>
 #include <unordered_map>
+#include <utility>
 #include <vector>
 
 #include "pp_common.h"
@@ -179,6 +181,16 @@ struct DiaArgs {
   int accumulate;       // dst_out = (accumulate ? dst_in : 0) + addend + alpha * sum
 };
 
+template <class F, int... R>
+__device__ __forceinline__ void for_rows_of(F&& f, std::integer_sequence<int, R...>) {
+  (f(std::integral_constant<int, R>{}), ...);
+}
+// f(0), ..., f(NR - 1) with compile-time arguments
+template <int NR, class F>
+__device__ __forceinline__ void for_rows(F&& f) {
+  for_rows_of(f, std::make_integer_sequence<int, NR>{});
+}
+
 // COMPACT: kMixed, some term is stored compactly; kSymmetric, all are and keep half the diagonals (the
 // offsets then are the same for every tuple).  Their values are read again soon (as a mirror image, or by
 // another fibre), so they are left in the caches instead of streamed past them.  Helium's full H in
@@ -201,8 +213,7 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
   C* xw = xs[wave];
   for (int j = lane; j < WIN; j += 64) xw[j] = cz<C>();
   C acc[NR];
-#pragma unroll
-  for (int r = 0; r < NR; ++r) acc[r] = cz<C>();
+  for_rows<NR>([&](auto r) { acc[r] = cz<C>(); });
   // One row per lane and symmetric bands throughout: element (i, i + k) is used where it is read, for
   // row i with x_{i+k} and for row i + k with lane i's own x_i.  The shift by k is the same for all
   // tuples, so those products gather in an accumulator per k and move to their rows once, at the end:
@@ -223,44 +234,51 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
   auto tuple = [&](int l) {
     return make_int4(from_lane(tup_l.x, l), from_lane(tup_l.y, l), from_lane(tup_l.z, l), 0);
   };
-  // a tuple's source values and its rows' bands (lanes past the fibre repeat its last row)
-  auto load = [&](const int4& tp, C (&x)[NR], V (&v)[NR][BW]) {
+  // (by components: an array of whole values copied from memory and on to LDS was kept in scratch memory,
+  // 23 us instead of 7 for 8 x 40 x 96 with 3 diagonals)
+  // source values of a tuple, and the bands of its row r per lane (lanes past the fibre repeat its last row)
+  auto load_x = [&](const int4& tp, C (&x)[NR]) {
+    const C* xp = a.src + (long long)tp.x * n;
+    for_rows<NR>([&](auto r) {
+      const C& v = xp[min(lane + 64 * r, n - 1)];
+      x[r].x = v.x;
+      x[r].y = v.y;
+    });
+  };
+  auto load_row = [&](const int4& tp, int r, V (&v)[BW]) {
     const int term = tp.z >> 1;
     const bool sym = COMPACT == kSymmetric || (COMPACT == kMixed && (a.sym >> term & 1));
-    const C* xp = a.src + (long long)tp.x * n;
     const unsigned long long base = (unsigned)from_lane((int)(dia_l & 0xffffffffu), term) |
                                     (unsigned long long)(unsigned)from_lane((int)(dia_l >> 32), term) << 32;
     const int fibre = (sym ? HB + 1 : BW) * n;  // stored values of a potential fibre
     const __amdgpu_buffer_rsrc_t band = __builtin_amdgcn_make_buffer_rsrc(
         reinterpret_cast<void*>(base + (unsigned long long)tp.y * fibre * sizeof(V)), (short)0,
         fibre * (int)sizeof(V), 0x00020000);
+    const int i = lane + 64 * r;
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int i = lane + 64 * r;
-      x[r] = xp[min(i, n - 1)];
+    for (int k = 0; k <= HB; ++k)
 #pragma unroll
-      for (int k = 0; k <= HB; ++k)
-#pragma unroll
-        for (int m = 0; m < (k && !SCATTER ? 2 : 1); ++m) {  // a diagonal and its mirror image, whose lines are the same
-          const int d = m ? HB - k : HB + k;
-          // stored diagonal of element (i, i + d - HB); of a mirrored one the row is i - (HB - d), and
-          // rows outside the matrix, like lanes past the fibre, are masked by an offset past the buffer
-          const int first = sym && m ? k : 0;
-          const int off = (sym ? k : d) * n - first;
-          v[r][d] =
-              ld_band<V, COMPACT != 0>(band, i < n && i >= first ? i * (int)sizeof(V) : kPastBand, off * (int)sizeof(V));
-        }
-    }
+      for (int m = 0; m < (k && !SCATTER ? 2 : 1); ++m) {  // a diagonal and its mirror image, whose lines are the same
+        const int d = m ? HB - k : HB + k;
+        // stored diagonal of element (i, i + d - HB); of a mirrored one the row is i - (HB - d), and
+        // rows outside the matrix, like lanes past the fibre, are masked by an offset past the buffer
+        const int first = sym && m ? k : 0;
+        const int off = (sym ? k : d) * n - first;
+        v[d] = ld_band<V, COMPACT != 0>(band, i < n && i >= first ? i * (int)sizeof(V) : kPastBand, off * (int)sizeof(V));
+      }
   };
-  auto use = [&](const int4& tp, const C (&x)[NR], const V (&v)[NR][BW]) {
+  auto window = [&](const C (&x)[NR]) {
+    for_rows<NR>([&](auto r) {
+      if (lane + 64 * r < n) {
+        xw[HB + lane + 64 * r].x = x[r].x;
+        xw[HB + lane + 64 * r].y = x[r].y;
+      }
+    });
+    wave_sync();
+  };
+  auto use_row = [&](const int4& tp, auto r, const C& x, const V (&v)[BW]) {
     const int term = tp.z >> 1;
     const bool cj = tp.z & 1;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int i = lane + 64 * r;
-      if (i < n) xw[HB + i] = x[r];
-    }
-    wave_sync();
     C s;
     if constexpr (sizeof(C) == sizeof(double2)) {
       s.x = __hiloint2double(from_lane(__double2hiint(scale_l.x), term), from_lane(__double2loint(scale_l.x), term));
@@ -269,26 +287,22 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
       s.x = __int_as_float(from_lane(__float_as_int(scale_l.x), term));
       s.y = __int_as_float(from_lane(__float_as_int(scale_l.y), term));
     }
+    const int i = lane + 64 * r;
+    C part = cz<C>();
+    if constexpr (SCATTER) {
+      C sx = cz<C>();
+      acc_scaled(sx, s, x);
+      acc_vx(part, v[HB], x, cj);
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int i = lane + 64 * r;
-      C part = cz<C>();
-      if constexpr (SCATTER) {
-        C sx = cz<C>();
-        acc_scaled(sx, s, x[r]);
-        acc_vx(part, v[r][HB], x[r], cj);
-#pragma unroll
-        for (int k = 1; k <= NK; ++k) {
-          acc_vx(part, v[r][HB + k], xw[i + HB + k], cj);
-          acc_vx(below[k], v[r][HB + k], sx, cj);
-        }
-      } else {
-#pragma unroll
-        for (int d = 0; d < BW; ++d) acc_vx(part, v[r][d], xw[i + d], cj);
+      for (int k = 1; k <= NK; ++k) {
+        acc_vx(part, v[HB + k], xw[i + HB + k], cj);
+        acc_vx(below[k], v[HB + k], sx, cj);
       }
-      acc_scaled(acc[r], s, part);
+    } else {
+#pragma unroll
+      for (int d = 0; d < BW; ++d) acc_vx(part, v[d], xw[i + d], cj);
     }
-    wave_sync();
+    acc_scaled(acc[r], s, part);
   };
   for (int b0 = w0; b0 < w1; b0 += 64) {
     const int last = min(64, w1 - b0) - 1;
@@ -296,6 +310,15 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
     if constexpr (NR * BW * sizeof(V) <= 13 * sizeof(double)) {
       // the next tuple's loads are issued before the current one is used: a wave waits for memory about
       // half as often, for one more set of registers
+      auto load = [&](const int4& tp, C (&x)[NR], V (&v)[NR][BW]) {
+        load_x(tp, x);
+        for_rows<NR>([&](auto r) { load_row(tp, r, v[r]); });
+      };
+      auto use = [&](const int4& tp, const C (&x)[NR], const V (&v)[NR][BW]) {
+        window(x);
+        for_rows<NR>([&](auto r) { use_row(tp, r, x[r], v[r]); });
+        wave_sync();
+      };
       C xa[NR], xb[NR];
       V va[NR][BW], vb[NR][BW];
       int4 ta = tuple(0), tb;
@@ -310,12 +333,25 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
         use(tb, xb, vb);
       }
     } else {
-      C x[NR];
-      V v[NR][BW];
+      // A row per lane at a time, the next one's bands loaded ahead: the bands of all rows at once take up
+      // to 512 registers and scratch memory, and leave one wave to a SIMD.  3 x 24 x 512, all pairs, 21
+      // diagonals: real 132 us (214 all at once, 192 by row without the next), complex 208 (777, 239);
+      // 4 x 30 x 300, 13 diagonals: 68 (109, 88) and 97 (158, 103).
+      constexpr int kAhead = BW * sizeof(V) <= 21 * sizeof(double) ? 1 : 0;  // rows loaded ahead
       for (int l = 0; l <= last; ++l) {
         const int4 tp = tuple(l);
-        load(tp, x, v);
-        use(tp, x, v);
+        C x[NR];
+        load_x(tp, x);
+        V v[kAhead + 1][BW];
+        load_row(tp, 0, v[0]);
+        window(x);
+        for_rows<NR>([&](auto r) {
+          constexpr int R = decltype(r)::value;
+          if constexpr (kAhead == 1 && R + 1 < NR) load_row(tp, R + 1, v[(R + 1) & 1]);
+          if constexpr (kAhead == 0 && R > 0) load_row(tp, R, v[0]);
+          use_row(tp, r, x[r], v[R & kAhead]);
+        });
+        wave_sync();
       }
     }
   }
@@ -331,8 +367,7 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
   }
   __syncthreads();
   C(*red)[WIN] = xs;
-#pragma unroll
-  for (int r = 0; r < NR; ++r) red[wave][lane + 64 * r] = acc[r];
+  for_rows<NR>([&](auto r) { red[wave][lane + 64 * r] = acc[r]; });
   __syncthreads();
   if (wave == 0) {
     C* out = a.dst + (long long)fib * n;
@@ -978,7 +1013,7 @@ void tp_run_f64(const TPPlanDevice& plan, const std::vector<const TPTerm*>& term
     a.sym = symmetric_terms(terms);
     if (!t0->is_real) launch_dia<double2, double2, kStreamed>(a, t0->bw, nr, blocks, s);
     else if (a.sym == (1u << terms.size()) - 1) launch_dia<double, double2, kSymmetric>(a, t0->bw, nr, blocks, s);
-  else if (any_compact(terms)) launch_dia<double, double2, kMixed>(a, t0->bw, nr, blocks, s);
+    else if (any_compact(terms)) launch_dia<double, double2, kMixed>(a, t0->bw, nr, blocks, s);
     else launch_dia<double, double2, kStreamed>(a, t0->bw, nr, blocks, s);
   } else {
     GenArgs<double2> a{};
