@@ -35,7 +35,6 @@
 #include <cstring>
 #include <numeric>
 #include <type_traits>
-#include <unordered_map>
 #include <utility>
 #include <vector>
 
@@ -721,10 +720,13 @@ __global__ void asymmetric_kernel(const double* __restrict__ dia, long long fibr
   if (__any(differs) && (threadIdx.x & 63) == 0) atomicOr(flag, 1ull);
 }
 
-// hash[f] of the bits of rows [first, first + len) of fibre f: one wave per fibre, a sum over its
-// values of a multiplicative mix of (bits, position)
+// Enters fibre f into a hash table (keys zero where empty, at least twice as many slots as fibres) under
+// the bits of its rows [first, first + len): slot[f] is its slot, owner[slot] the smallest fibre there.
+// One wave per fibre; the hash is a sum over its values of SplitMix64's finaliser (G. L. Steele, D. Lea,
+// C. H. Flood, OOPSLA 2014) of (bits, position).
 __global__ __launch_bounds__(256) void fibre_hash_kernel(const double* __restrict__ dia, long long fibres, int stride,
-                                                         int first, int len, unsigned long long* __restrict__ hash) {
+                                                         int first, int len, unsigned long long mask,
+                                                         unsigned long long* keys, int* owner, int* __restrict__ slot) {
   const long long f = blockIdx.x * 4LL + (threadIdx.x >> 6);
   if (f >= fibres) return;
   const double* v = dia + f * stride + first;
@@ -736,19 +738,28 @@ __global__ __launch_bounds__(256) void fibre_hash_kernel(const double* __restric
     h += w ^ (w >> 31);
   }
   for (int off = 32; off > 0; off >>= 1) h += __shfl_down(h, off, 64);
-  if ((threadIdx.x & 63) == 0) hash[f] = h;
+  if ((threadIdx.x & 63) != 0) return;
+  if (h == 0) h = 1;
+  unsigned long long i = h & mask;
+  for (unsigned long long old; (old = atomicCAS(&keys[i], 0ull, h)) != 0 && old != h;) i = (i + 1) & mask;
+  atomicMin(&owner[i], (int)f);
+  slot[f] = (int)i;
 }
 
-// flag |= fibre f differs in its bits from fibre rep[f]
+// rep[f] (slot[f] on entry) = the first fibre of f's slot; flag |= they differ in their bits
 __global__ __launch_bounds__(256) void fibre_differs_kernel(const double* __restrict__ dia, long long fibres, int stride,
-                                                            int first, int len, const int* __restrict__ rep,
+                                                            int first, int len, const int* __restrict__ owner, int* rep,
                                                             unsigned long long* flag) {
   const long long f = blockIdx.x * 4LL + (threadIdx.x >> 6);
-  if (f >= fibres || rep[f] == f) return;
-  const double *a = dia + f * stride + first, *b = dia + (long long)rep[f] * stride + first;
+  if (f >= fibres) return;
+  const int r = owner[rep[f]];
+  const double *a = dia + f * stride + first, *b = dia + (long long)r * stride + first;
   bool differs = false;
-  for (int k = threadIdx.x & 63; k < len; k += 64) differs |= __double_as_longlong(a[k]) != __double_as_longlong(b[k]);
+  if (r != f)
+    for (int k = threadIdx.x & 63; k < len; k += 64)
+      differs |= __double_as_longlong(a[k]) != __double_as_longlong(b[k]);
   if (__any(differs) && (threadIdx.x & 63) == 0) atomicOr(flag, 1ull);
+  if ((threadIdx.x & 63) == 0) rep[f] = r;
 }
 
 // out[u] = rows [first, first + len) of fibre kept[u]
@@ -761,67 +772,68 @@ __global__ __launch_bounds__(256) void gather_fibres_kernel(const double* __rest
   for (int k = threadIdx.x & 63; k < len; k += 64) out[u * len + k] = v[k];
 }
 
+// Values of a term from which compact storage is looked for: the search costs 0.1 ms a term, and a
+// smaller term is read from L2 in any case (hydrogen, 8 x 120: set-up 0.25 ms without it, 0.42 with; the
+// same product).  5 x 12 x 12 helium, of 40000 values and more a term, gains: 10 us of a product's 23.
+constexpr long long kCompactFrom = 1 << 15;
+
 // Stores a real banded term compactly where that saves at least a quarter (a hash collision keeps it
-// as it is: equality is checked value by value).
+// as it is: equality is checked value by value).  The table is built on the device: setting up helium's
+// three terms (425000 fibres, 2.65 GB) takes 16.9 ms, 16.0 without the search and 24.7 with the table on
+// the host.
 static void compact_term(TPTerm& term, long long pfib, int n, hipStream_t s) {
-  if (pfib >= (1ll << 31)) return;
+  if (pfib >= (1ll << 30)) return;  // (the table's slots are ints)
   const int bw = term.bw, hb = (bw - 1) / 2, stride = bw * n;
   const int wave_blocks = ceil_div(pfib, 4);
-  DeviceBuffer<unsigned long long> flag(1), hash(pfib);
+  // one allocation for the search: a flag, the table's keys and owners, and an index per fibre
+  size_t slots = 64;
+  while (slots < 2 * (size_t)pfib) slots *= 2;
+  DeviceBuffer<unsigned long long> scratch(1 + slots + (slots + pfib + 1) / 2);
+  unsigned long long *flag = scratch.ptr, *keys = flag + 1;
+  int *owner = reinterpret_cast<int*>(keys + slots), *index = owner + slots;
+  PP_HIP(hipMemsetAsync(flag, 0, (1 + slots) * sizeof(unsigned long long), s));
+  PP_HIP(hipMemsetAsync(owner, 0x7f, slots * sizeof(int), s));
   auto read_flag = [&]() {
     unsigned long long h = 0;
-    PP_HIP(hipMemcpyAsync(&h, flag.ptr, sizeof(h), hipMemcpyDeviceToHost, s));
+    PP_HIP(hipMemcpyAsync(&h, flag, sizeof(h), hipMemcpyDeviceToHost, s));
     PP_HIP(hipStreamSynchronize(s));
     return h != 0;
   };
   bool sym = hb > 0;
   if (sym) {
-    PP_HIP(hipMemsetAsync(flag.ptr, 0, sizeof(unsigned long long), s));
     const long long total = pfib * hb * (long long)n;
     hipLaunchKernelGGL(asymmetric_kernel, dim3((int)std::min<long long>(65536, (total + 255) / 256)), dim3(256), 0, s,
-                       term.dia_real.ptr, pfib, n, bw, flag.ptr);
+                       term.dia_real.ptr, pfib, n, bw, flag);
     PP_HIP(hipGetLastError());
     sym = !read_flag();
+    if (!sym) PP_HIP(hipMemsetAsync(flag, 0, sizeof(unsigned long long), s));
   }
   const int first = sym ? hb * n : 0, len = sym ? (hb + 1) * n : stride;
   hipLaunchKernelGGL(fibre_hash_kernel, dim3(wave_blocks), dim3(256), 0, s, term.dia_real.ptr, pfib, stride, first, len,
-                     hash.ptr);
+                     (unsigned long long)(slots - 1), keys, owner, index);
+  hipLaunchKernelGGL(fibre_differs_kernel, dim3(wave_blocks), dim3(256), 0, s, term.dia_real.ptr, pfib, stride, first,
+                     len, owner, index, flag);
   PP_HIP(hipGetLastError());
-  std::vector<unsigned long long> h(pfib);
-  PP_HIP(hipMemcpyAsync(h.data(), hash.ptr, pfib * sizeof(h[0]), hipMemcpyDeviceToHost, s));
-  PP_HIP(hipStreamSynchronize(s));
-  std::unordered_map<unsigned long long, int> seen;
-  seen.reserve(pfib);
   std::vector<int> canon(pfib), rep(pfib), kept;
-  for (long long f = 0; f < pfib; ++f) {
-    const auto it = seen.emplace(h[f], (int)kept.size());
-    if (it.second) kept.push_back((int)f);
-    canon[f] = it.first->second;
-    rep[f] = kept[canon[f]];
+  PP_HIP(hipMemcpyAsync(rep.data(), index, pfib * sizeof(int), hipMemcpyDeviceToHost, s));
+  bool merged = !read_flag();
+  for (long long f = 0; merged && f < pfib; ++f) {  // rep[f] <= f
+    canon[f] = rep[f] == f ? (int)kept.size() : canon[rep[f]];
+    if (rep[f] == f) kept.push_back((int)f);
   }
-  bool merged = kept.size() < (size_t)pfib;
-  if (merged) {
-    DeviceBuffer<int> reps;
-    reps.upload(rep.data(), rep.size(), s);
-    PP_HIP(hipMemsetAsync(flag.ptr, 0, sizeof(unsigned long long), s));
-    hipLaunchKernelGGL(fibre_differs_kernel, dim3(wave_blocks), dim3(256), 0, s, term.dia_real.ptr, pfib, stride, first,
-                       len, reps.ptr, flag.ptr);
-    PP_HIP(hipGetLastError());
-    if (read_flag()) merged = false;
-  }
+  merged = merged && kept.size() < (size_t)pfib;
   if (!merged) {
     kept.resize(pfib);
     std::iota(kept.begin(), kept.end(), 0);
   }
   const long long size = (long long)kept.size() * len;
   if (size * 4 > pfib * (long long)stride * 3) return;
-  DeviceBuffer<int> keep;
-  keep.upload(kept.data(), kept.size(), s);
   DeviceBuffer<double> out(size);
+  PP_HIP(hipMemcpyAsync(index, kept.data(), kept.size() * sizeof(int), hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(gather_fibres_kernel, dim3(ceil_div((long long)kept.size(), 4)), dim3(256), 0, s,
-                     term.dia_real.ptr, (long long)kept.size(), stride, first, len, keep.ptr, out.ptr);
+                     term.dia_real.ptr, (long long)kept.size(), stride, first, len, index, out.ptr);
   PP_HIP(hipGetLastError());
-  PP_HIP(hipStreamSynchronize(s));  // before the buffers that the copy reads are released
+  PP_HIP(hipStreamSynchronize(s));  // before what the copy reads is released
   std::swap(term.dia_real.ptr, out.ptr);
   std::swap(term.dia_real.count, out.count);
   term.sym = sym;
@@ -897,7 +909,7 @@ void tp_create_impl(int rank, const int* ids, const double2* potential, const in
       term.stream_bytes = total * (long long)sizeof(double2);
     }
     PP_HIP(hipGetLastError());
-    if (compact && term.is_real) compact_term(term, pfib, n, s);
+    if (compact && term.is_real && total >= kCompactFrom) compact_term(term, pfib, n, s);
   } else {
     term.dia = false;
     term.vref.resize(pcount);

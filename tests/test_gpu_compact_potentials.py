@@ -47,6 +47,18 @@ def _potential(rng, nc, n1, b1, n2, b2, kind):
     return TensorPotentialData(kind, geo, data), dense
 
 
+def _outer(n2, b2, least):
+    """Channels, rows and band of the outer ranks that give a term at least `least` stored values."""
+    for nc, n1, b1 in ((2, 3, 1), (3, 4, 2), (5, 5, 2), (6, 6, 2), (8, 8, 2), (16, 8, 2)):
+        pairs = sum(min(n1, a + b1 + 1) - max(0, a - b1) for a in range(n1))
+        if nc * nc * pairs * n2 * (2 * b2 + 1) >= least:
+            break
+    return nc, n1, b1
+
+
+COMPACT_FROM = 2 ** 15  # values from which compact storage is looked for
+
+
 @pytest.mark.parametrize("b2", range(11))
 @pytest.mark.parametrize("kinds", [("symmetric",), ("none",), ("complex",), ("symmetric", "none")], ids="+".join)
 @pytest.mark.parametrize("n2", [40, 100, 200, 260])
@@ -61,10 +73,14 @@ def test_hamiltonian_of_compact_terms(torch, kinds, n2, b2):
     _check_hamiltonian(torch, kinds, n2, b2)
 
 
-def _check_hamiltonian(torch, kinds, n2, b2):
+def test_small_terms_are_kept_as_they_are(torch):
+    _check_hamiltonian(torch, ("symmetric", "half"), 13, 4, least=0)
+
+
+def _check_hamiltonian(torch, kinds, n2, b2, least=COMPACT_FROM):
     from pyprop_amd.propagator import BasisPropagator, CombinedRepresentation, Wavefunction
     rng = np.random.default_rng(n2 + len(kinds))
-    nc, n1, b1 = (3, 4, 2) if n2 * b2 < 1000 else (2, 3, 1)
+    nc, n1, b1 = _outer(n2, b2, least)
     made = [_potential(rng, nc, n1, b1, n2, b2, k) for k in kinds]
     repr_ = CombinedRepresentation((nc, n1, n2), [None, None, None])
     x = rng.standard_normal((nc, n1, n2)) + 1j * rng.standard_normal((nc, n1, n2))
@@ -81,8 +97,10 @@ def _check_hamiltonian(torch, kinds, n2, b2):
         full = 8 * nc * nc * p.GeometryList[1].pair_count * (2 * b2 + 1) * n2
         if k in ("none", "complex"):
             assert p.stream_bytes == (full if k == "none" else 2 * full)
-        else:
-            assert p.stream_bytes < 0.76 * full or b2 == 0  # a diagonal has no mirror image
+        elif least == 0:
+            assert p.stream_bytes == full
+        elif b2 > 0:  # (a diagonal has no mirror image)
+            assert p.stream_bytes < 0.76 * full
     # one potential at a time, added to what is there
     for (data, dense), p in zip(made, base.PotentialList):
         acc = torch.ones_like(psi.data)
@@ -97,10 +115,12 @@ def test_fp32_multiply_of_compact_terms(torch, n2, b2):
     from pyprop_amd import _native as N, device as D
     from pyprop_amd.tensorpotential import TensorPotential
     rng = np.random.default_rng(n2)
-    data, dense = _potential(rng, 2, 4, 2, n2, b2, "symmetric")
-    p = TensorPotential(data, (2, 4, n2))
+    nc, n1, b1 = _outer(n2, b2, COMPACT_FROM)
+    data, dense = _potential(rng, nc, n1, b1, n2, b2, "symmetric")
+    p = TensorPotential(data, (nc, n1, n2))
     p.SetupStep()
-    x = rng.standard_normal((2, 4, n2)) + 1j * rng.standard_normal((2, 4, n2))
+    assert p.stream_bytes < 8 * 0.76 * data.data.size
+    x = rng.standard_normal((nc, n1, n2)) + 1j * rng.standard_normal((nc, n1, n2))
     src = torch.from_numpy(x).to("cuda").to(torch.complex64)
     dst = torch.zeros_like(src)
     N.check(N.load().pp_tp_multiply_f32(p.plan, C.c_float(1.0), D.ptr(src), D.ptr(dst), D.stream_handle()))
@@ -113,11 +133,15 @@ def test_nan_stays_in_the_rows_it_couples_to(torch):
     from pyprop_amd.propagator import BasisPropagator, CombinedRepresentation, Wavefunction
     rng = np.random.default_rng(1)
     for n2 in (40, 90):
-        data, _ = _potential(rng, 1, 1, 0, n2, 3, "symmetric")
-        repr_ = CombinedRepresentation((1, 1, n2), [None, None, None])
-        x = np.ones((1, 1, n2), complex)
-        x[0, 0, 20] = np.nan
+        nc, n1, b1 = _outer(n2, 3, COMPACT_FROM)
+        data, _ = _potential(rng, nc, n1, b1, n2, 3, "symmetric")
+        repr_ = CombinedRepresentation((nc, n1, n2), [None, None, None])
+        x = np.ones((nc, n1, n2), complex)
+        x[1, 0, 20] = np.nan
         psi, out = Wavefunction(repr_, x), Wavefunction(repr_)
-        BasisPropagator(psi, [data], consolidate=False).MultiplyHamiltonianNoOverlap(psi, out, 0.0)
-        bad = np.isnan(out.numpy()[0, 0].real)
-        assert np.array_equal(np.nonzero(bad)[0], np.arange(17, 24))
+        base = BasisPropagator(psi, [data], consolidate=False)
+        base.MultiplyHamiltonianNoOverlap(psi, out, 0.0)
+        assert base.PotentialList[0].stream_bytes < 8 * 0.76 * data.data.size
+        bad = np.argwhere(np.isnan(out.numpy().real))
+        expected = [(c, i, j) for c in range(nc) for i in range(b1 + 1) for j in range(17, 24)]
+        assert np.array_equal(bad, expected)
