@@ -654,6 +654,9 @@ static void xcd_order(TPPlanData& pd, int group) {
     std::stable_sort(p.begin(), p.end(), [&](int a, int b) { return weight[a / group] > weight[b / group]; });
     most = std::max(most, p.size());
   }
+  // (tuples gathered in few fibres: the other XCDs' ranges hold most fibres and the filling most
+  // workgroups; the order by length is kept)
+  if (most * kXcds > 2 * (size_t)pd.n_fibres + 64) return;
   pd.fib_order.assign(most * kXcds, -1);
   for (int x = 0; x < kXcds; ++x)
     for (size_t k = 0; k < part[x].size(); ++k) pd.fib_order[k * kXcds + x] = part[x][k];
@@ -782,7 +785,7 @@ constexpr long long kCompactFrom = 1 << 15;
 // three terms (425000 fibres, 2.65 GB) takes 16.9 ms, 16.0 without the search and 24.7 with the table on
 // the host.
 static void compact_term(TPTerm& term, long long pfib, int n, hipStream_t s) {
-  if (pfib >= (1ll << 30)) return;  // (the table's slots are ints)
+  if (pfib >= (1ll << 26)) return;  // a wave per fibre: a launch holds fewer than 2^32 threads
   const int bw = term.bw, hb = (bw - 1) / 2, stride = bw * n;
   const int wave_blocks = ceil_div(pfib, 4);
   // one allocation for the search: a flag, the table's keys and owners, and an index per fibre

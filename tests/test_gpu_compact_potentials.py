@@ -145,3 +145,55 @@ def test_nan_stays_in_the_rows_it_couples_to(torch):
         bad = np.argwhere(np.isnan(out.numpy().real))
         expected = [(c, i, j) for c in range(nc) for i in range(b1 + 1) for j in range(17, 24)]
         assert np.array_equal(bad, expected)
+
+
+def test_uneven_fibres(torch):
+    """One destination fibre with nearly all tuples: the launch order by XCDs would be mostly empty."""
+    from pyprop_amd.geometry import Geometry
+    from pyprop_amd.propagator import BasisPropagator, CombinedRepresentation, Wavefunction
+    from pyprop_amd.systems import TensorPotentialData
+    rng = np.random.default_rng(5)
+    nc, n, b, repeats = 300, 8, 2, 40
+    pairs0 = np.array([(0, c) for c in range(nc)] * repeats + [(c, c) for c in range(1, nc)], dtype=np.int32)
+    pairs1 = np.array([(i, j) for j in range(n) for i in range(j - b, j + b + 1)], dtype=np.int32)
+    inside = (pairs1[:, 0] >= 0) & (pairs1[:, 0] < n)
+    band = np.add.outer(np.arange(n), np.arange(n)) / 4.0
+    row = np.where(inside, band[pairs1[:, 0] * inside, pairs1[:, 1]], 0.0)
+    amp = rng.integers(1, 5, len(pairs0)) / 4.0
+    data = TensorPotentialData("uneven", [Geometry("Simp", pairs0, False, nc),
+                                          Geometry("BandNH", np.where(inside[:, None], pairs1, 0), True, n)],
+                               (amp[:, None] * row).astype(complex))
+    x = rng.standard_normal((nc, n)) + 1j * rng.standard_normal((nc, n))
+    repr_ = CombinedRepresentation((nc, n), [None, None])
+    psi, out = Wavefunction(repr_, x), Wavefunction(repr_)
+    base = BasisPropagator(psi, [data], consolidate=False)
+    assert base.PotentialList[0].stream_bytes < 8 * 0.1 * data.data.size  # four amplitudes
+    base.MultiplyHamiltonianNoOverlap(psi, out, 0.0)
+    M = band * (np.abs(np.subtract.outer(np.arange(n), np.arange(n))) <= b)
+    A = np.zeros((nc, nc))
+    np.add.at(A, (pairs0[:, 0], pairs0[:, 1]), amp)
+    ref = A @ x @ M.T
+    bound = 2.0 ** -53 * (len(pairs0) * (2 * b + 1) + 4) * (A @ np.abs(x) @ M.T)
+    assert np.all(np.abs(out.numpy() - ref) <= bound)
+
+
+def test_more_fibres_than_a_launch_has_waves(torch):
+    """8195 x 8195 channels of one row, over 2^26 potential fibres: kept as they are."""
+    from pyprop_amd.geometry import Geometry
+    from pyprop_amd.systems import TensorPotentialData
+    from pyprop_amd.tensorpotential import TensorPotential
+    nc = 8195
+    a = np.arange(nc, dtype=np.int32)
+    pairs = np.stack(np.broadcast_arrays(a[:, None], a[None, :]), -1).reshape(-1, 2)
+    u, w = 1.0 + a % 7, 2.0 + a % 5
+    data = TensorPotentialData("one row", [Geometry("Simp", pairs, False, nc),
+                                           Geometry("BandNH", np.zeros((1, 2), np.int32), True, 1)],
+                               np.multiply.outer(u, w).astype(complex).reshape(-1, 1))
+    p = TensorPotential(data, (nc, 1))
+    p.SetupStep()
+    assert p.stream_bytes == 8 * nc * nc
+    x = torch.from_numpy(np.arange(nc) % 3 + 1j * (np.arange(nc) % 4)).to("cuda").reshape(nc, 1)
+    out = torch.zeros_like(x)
+    p.MultiplyPotential(x, out, 0.0)
+    # whole numbers below 2^53: exact
+    assert np.array_equal(out.cpu().numpy()[:, 0], u * (w @ x.cpu().numpy()[:, 0]))
