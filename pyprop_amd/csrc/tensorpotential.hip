@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <array>
 #include <cstring>
+#include <new>
 #include <numeric>
 #include <type_traits>
 #include <utility>
@@ -912,7 +913,17 @@ void tp_create_impl(int rank, const int* ids, const double2* potential, const in
       term.stream_bytes = total * (long long)sizeof(double2);
     }
     PP_HIP(hipGetLastError());
-    if (compact && term.is_real && total >= kCompactFrom) compact_term(term, pfib, n, s);
+    if (compact && term.is_real && total >= kCompactFrom) {
+      // Without room for the search or the second copy the term is kept as it is (compact_term changes it
+      // at its end only).
+      try {
+        compact_term(term, pfib, n, s);
+      } catch (const Error& e) {
+        if (e.code != PP_ERR_ALLOC) throw;
+        (void)hipGetLastError();  // or the next launch's check would report the failed allocation
+      } catch (const std::bad_alloc&) {
+      }
+    }
   } else {
     term.dia = false;
     term.vref.resize(pcount);

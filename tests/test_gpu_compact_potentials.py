@@ -197,3 +197,39 @@ def test_more_fibres_than_a_launch_has_waves(torch):
     p.MultiplyPotential(x, out, 0.0)
     # whole numbers below 2^53: exact
     assert np.array_equal(out.cpu().numpy()[:, 0], u * (w @ x.cpu().numpy()[:, 0]))
+
+
+def test_without_room_for_a_second_copy(torch):
+    """A potential that fits the device once but not once and a half is kept as it is."""
+    import ctypes as C
+    from pyprop_amd import _native as N, device as D
+    nc, n, b = 1600, 40, 2
+    values = nc * nc * n * (2 * b + 1)  # 512 million, 4 GB stored
+    a = np.arange(nc, dtype=np.int32)
+    pairs = np.ascontiguousarray(np.stack(np.broadcast_arrays(a[:, None], a[None, :]), -1).reshape(-1, 2))
+    pot = torch.zeros((nc * nc, n, 2 * b + 1), dtype=torch.complex128, device="cuda")
+    pot.real[:, :, b] = torch.arange(nc * nc, dtype=torch.float64, device="cuda")[:, None]  # all different
+    x = torch.ones((nc, n), dtype=torch.complex128, device="cuda")
+    out = torch.zeros_like(x)
+    want = pot.real[:, 0, b].reshape(nc, nc).sum(1)  # whole numbers: exact
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    hog = torch.empty(max(0, torch.cuda.mem_get_info()[0] - 8 * values - (1 << 30)), dtype=torch.uint8, device="cuda")
+    h = C.c_void_p()
+    ids = np.array([N.STORAGE["Simp"], N.STORAGE["BandNH"]], dtype=np.int32)
+    ext, src = np.array([nc * nc, n * (2 * b + 1)], dtype=np.int32), np.array([nc, n], dtype=np.int32)
+    lists, counts = (C.c_void_p * 2)(pairs.ctypes.data, None), np.array([nc * nc, 0], dtype=np.int32)
+    lib = N.load()
+    N.check(lib.pp_tp_create(2, D.hptr(ids), D.ptr(pot), D.hptr(ext), D.hptr(src), C.cast(lists, C.c_void_p),
+                             D.hptr(counts), D.stream_handle(), C.byref(h)))
+    del hog
+    try:
+        nbytes = C.c_int64()
+        N.check(lib.pp_tp_info(h, C.byref(nbytes), None, None, None))
+        assert nbytes.value == 8 * values
+        N.check(lib.pp_tp_multiply(h, 1.0, D.ptr(x), D.ptr(out), D.stream_handle()))
+        assert torch.equal(out.real, want[:, None].expand(nc, n)) and not out.imag.any()
+    finally:
+        lib.pp_tp_destroy(h)
+        del pot
+        torch.cuda.empty_cache()
