@@ -867,13 +867,13 @@ static int sym_form(const Precond& pc) {
   return (pc.b * pc.n2 + 63) / 64 * 32 + (pc.b <= 4 ? 9 : pc.b <= 6 ? 13 : 17);
 }
 
+// The LDS limit belongs to the kernel, not to a preconditioner: the most that any of this form needs.
 static void sym_prepare(const Precond& pc) {
-  const int nt = (pc.b * pc.n2 + 63) / 64;
   switch (sym_form(pc)) {
 #define PP_SYM(NT, W)                                                                                          \
   case NT * 32 + W:                                                                                            \
     PP_HIP(hipFuncSetAttribute((const void*)pc_sym_kernel<NT, W>, hipFuncAttributeMaxDynamicSharedMemorySize,  \
-                               (int)sym_lds(nt, pc.n2, pc.b)));                                                \
+                               (int)sym_lds(NT, 64, W / 2)));                                                  \
     break;
     PP_SYM_FORMS(PP_SYM)
 #undef PP_SYM

@@ -30,7 +30,7 @@ def _pairs(n, b):
     return np.array([(i, j) for i in range(n) for j in range(max(0, i - b), min(n, i + b + 1))], dtype=np.int32)
 
 
-def _check(torch, nchan, n1, n2, b, kind, sh, ss, seed=0):
+def _check(torch, nchan, n1, n2, b, kind, sh, ss, seed=0, before_solve=None):
     from pyprop_amd import _native as N, device as D
     rng = np.random.default_rng(seed)
     S1, S2 = _band(rng, n1, b), _band(rng, n2, b)
@@ -46,6 +46,8 @@ def _check(torch, nchan, n1, n2, b, kind, sh, ss, seed=0):
     h = C.c_void_p()
     N.check(N.load().pp_precond_create(nchan, n1, n2, b, D.hptr(S1), D.hptr(S2), D.hptr(P), len(p1), D.hptr(p1), len(p2),
                                        D.hptr(p2), N.cplx(sh), N.cplx(ss), C.byref(h)))
+    if before_solve:
+        before_solve()
     x = rng.standard_normal((nchan, n1, n2)) + 1j * rng.standard_normal((nchan, n1, n2))
     t = torch.from_numpy(x.copy()).to("cuda")
     guard = t.clone()
@@ -63,14 +65,21 @@ def _check(torch, nchan, n1, n2, b, kind, sh, ss, seed=0):
         assert err < 1e-14 * np.linalg.cond(M) * 4, (c, err)
 
 
-# one to ten superblocks, a short last one, one to eight column tiles of 64
-SIZES = [(2, 1, 1), (5, 3, 1), (7, 7, 6), (9, 64, 8), (12, 10, 6), (13, 13, 4), (19, 21, 5), (20, 33, 2), (24, 40, 6),
-         (16, 64, 7)]
+# two to ten superblocks, a short last one, each band limit (4, 6, 8) with each of its counts of 64-column tiles
+SIZES = [(2, 1, 1), (5, 3, 1), (13, 13, 4), (20, 33, 2), (7, 64, 3), (9, 49, 4), (7, 7, 6), (12, 10, 6), (19, 21, 5),
+         (11, 29, 5), (24, 40, 6), (13, 64, 5), (13, 60, 6), (9, 9, 7), (16, 16, 8), (17, 24, 8), (15, 32, 8), (16, 40, 8),
+         (15, 54, 7), (16, 64, 7), (9, 64, 8)]
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
 def test_symmetric_superblocks(torch, size):
     _check(torch, 3 if size[0] * size[1] < 700 else 1, *size, "symmetric", 0.3j, 1.0, seed=size[0])
+
+
+def test_a_smaller_preconditioner_of_the_same_form_in_between(torch):
+    """74 KB of LDS; the one that is created before the solve needs 73 KB."""
+    _check(torch, 1, 12, 64, 6, "symmetric", 0.3j, 1.0,
+           before_solve=lambda: _check(torch, 1, 12, 54, 6, "symmetric", 0.3j, 1.0))
 
 
 @pytest.mark.parametrize("kind", ["unsymmetric", "complex"])
