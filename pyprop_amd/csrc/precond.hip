@@ -940,7 +940,7 @@ extern "C" int pp_precond_create(int nchan, int n1, int n2, int band, const doub
     }
     const cd sh(scaling_h.re, scaling_h.im), ss(scaling_s.re, scaling_s.im);
     const cd* pd = reinterpret_cast<const cd*>(p_data);
-    const unsigned nthreads = std::max(1u, std::min<unsigned>(std::thread::hardware_concurrency(), 16u));
+    const unsigned nthreads = std::max(1u, std::min({std::thread::hardware_concurrency(), 16u, (unsigned)nchan}));
     auto each_channel = [&](auto&& work) {
       std::vector<std::thread> pool;
       std::vector<std::string> errors(nthreads);
