@@ -307,9 +307,9 @@ typedef struct pp_precond pp_precond;
  *   s1, s2: host dense (n1, n1), (n2, n2) overlaps; band = half bandwidth of S (k-1).
  *   p_data: host complex (nchan, p1_count, p2_count) angular-diagonal potential with
  *   Simp pair lists pairs1 (p1_count, 2) and pairs2 (p2_count, 2) for the radial ranks.
- * No pivoting (the real part of M_c is positive definite); the SuperLU variant of the
- * reference solves the same systems exactly.  Real symmetric S and P with n2 <= 64 and
- * band <= 8 are factorized in superblocks of band block rows, everything else as a block LU. */
+ * No pivoting; the SuperLU variant of the reference solves the same systems exactly.  Real
+ * symmetric S and P with n2 <= 64 and band <= 8, of which some multiple has a definite Hermitian
+ * part, are factorized in superblocks of band block rows, everything else as a block LU. */
 int pp_precond_create(int nchan, int n1, int n2, int band, const double* s1, const double* s2,
                       const pp_cplx* p_data, int p1_count, const int32_t* pairs1, int p2_count,
                       const int32_t* pairs2, pp_cplx scaling_h, pp_cplx scaling_s,

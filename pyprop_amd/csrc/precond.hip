@@ -7,8 +7,9 @@
 //
 // M_c is block banded: n2 x n2 blocks (I, J) with |I - J| <= b (b = B-spline order - 1).
 //
-// Symmetric M_c (real symmetric S and P: every Hamiltonian of this library), b n2 <= 512: b block
-// rows together form a superblock s of m = b n2 unknowns, and M_c is block tridiagonal in them with
+// Symmetric M_c (real symmetric S and P: every Hamiltonian of this library) of which some multiple has a
+// definite Hermitian part (S x S + i dt/2 P_c; H - sigma S for sigma below the spectrum), b n2 <= 512: b
+// block rows together form a superblock s of m = b n2 unknowns, and M_c is block tridiagonal in them with
 // the sparse couplings A_s,s+1 (S and P entries).  Superblocks are eliminated from both ends towards
 // the middle one; with the pivot blocks D_s = A_ss - A_s,s-+1 D_s-+1^-1 A_s-+1,s inverted on the host
 //   w_s = D_s^-1 (b_s - A_s,s-+1 w_s-+1)      from the ends inwards (two chains at once)
@@ -18,9 +19,7 @@
 // (10 superblocks of 360), against 0.87 GB of L' or U' in the general form below, by two workgroups
 // per channel instead of one, in 10 steps instead of 60.  See pc_sym_kernel for the figures.
 //
-// Otherwise the host factors it once per channel by a right-looking block LU without pivoting
-// (the Hermitian part of M_c is positive definite: S x S is, and scaling_h P_c is
-// i dt/2 times a real symmetric matrix), and stores for each block row I
+// Otherwise the host factors it once per channel by a right-looking block LU without pivoting, and stores for each block row I
 //   L_II^-1,  L'_IJ = L_II^-1 L_IJ (J = I-b..I-1),  U_II^-1,  U'_IJ = U_II^-1 U_IJ.
 // The device solve is then
 //   c_I = L_II^-1 b_I        (all I in parallel)
@@ -30,6 +29,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <complex>
 #include <limits>
@@ -226,13 +226,30 @@ static void split_gemm_sub(int n, const SplitBlock& A, bool at, const SplitBlock
   }
 }
 
-// A <- A^-1 (n x n), Gauss-Jordan without pivoting
-static void split_invert(int n, SplitBlock& A) {
+// The directions of an elimination's pivots in the complex plane, relative to the first diagonal entry.
+// Without pivoting the elimination is stable where they stay well within a half plane: where some multiple of M
+// has a definite Hermitian part, so has every Schur complement.  Otherwise (sigma inside the spectrum) the
+// superblocks' explicit inverses lose more digits than the block LU: 20 x 20 with band 5, random symmetric
+// P + 0.3 S: error 1.5e-8, with the block LU 4.9e-11 (S + 0.3i P: 6.0e-16 and 5.4e-16).
+struct PivotFan {
+  cd ref;
+  double lo = 0.0, hi = 0.0;
+  static constexpr double kWidest = 2.1;  // 120 degrees; a Crank-Nicolson step's span just over 90
+  bool add(cd piv) {  // false: zero, not a number, or too far from the others
+    const double a = std::arg(piv * std::conj(ref));
+    lo = std::min(lo, a);
+    hi = std::max(hi, a);
+    return piv != cd(0) && std::isfinite(a) && hi - lo <= kWidest;
+  }
+};
+
+// A <- A^-1 (n x n), Gauss-Jordan without pivoting; false as soon as a pivot does not fit the others
+static bool split_invert(int n, SplitBlock& A, PivotFan& fan) {
   for (int k = 0; k < n; ++k) {
     double* kr = A.re.data() + (size_t)k * n;
     double* ki = A.im.data() + (size_t)k * n;
     const cd piv(kr[k], ki[k]);
-    if (piv == cd(0)) throw Error(PP_ERR_INVALID, "zero pivot in preconditioner block LU");
+    if (!fan.add(piv)) return false;
     const cd inv = 1.0 / piv;
     kr[k] = 1.0;
     ki[k] = 0.0;
@@ -253,6 +270,7 @@ static void split_invert(int n, SplitBlock& A) {
       }
     }
   }
+  return true;
 }
 
 // The entries of channel c's M_c, upper triangle in the radial indices.
@@ -290,8 +308,9 @@ static bool is_symmetric(const SymMatrix& M, int p1) {
   return true;
 }
 
-// Inverse pivot blocks of one channel into dinv [ns][m][m] (upper triangle, halved diagonal).
-static void factor_symmetric(const SymMatrix& M, int ns, int mid, cd* dinv) {
+// Inverse pivot blocks of one channel into dinv [ns][m][m] (upper triangle, halved diagonal); false, with
+// dinv unfinished, where the pivots spread too far.
+static bool factor_symmetric(const SymMatrix& M, int ns, int mid, cd* dinv) {
   const int n2 = M.n2, b = M.b, m = b * n2;
   const size_t bs = (size_t)n2 * n2;
   auto rows = [&](int s) { return std::min(b, M.n1 - s * b); };
@@ -302,6 +321,7 @@ static void factor_symmetric(const SymMatrix& M, int ns, int mid, cd* dinv) {
   std::vector<SplitBlock> D, W, Dl, Dr;  // blocks (q, q') of a pivot block, its inverse, the chains' last inverses
   SplitBlock scratch(bs), pivot(bs);
   std::vector<SplitBlock> panel(b, SplitBlock(bs));
+  PivotFan fan{M(0, 0, 0, 0)};
   // D -= A_s,f Dinv_f A_f,s with the sparse couplings A
   auto subtract = [&](int s, int f, const std::vector<SplitBlock>& inv) {
     const int rs = rows(s), rf = rows(f);
@@ -344,7 +364,7 @@ static void factor_symmetric(const SymMatrix& M, int ns, int mid, cd* dinv) {
       }
   };
   // D (upper blocks) <- D^-1 (all blocks), sweeping one block row after the other: D becomes -D^-1
-  auto invert = [&](int rs) {
+  auto invert = [&](int rs) {  // false: see split_invert
     for (int k = 0; k < rs; ++k) {
       pivot = D[k * b + k];
       // the pivot block is symmetric to rounding: use its upper triangle
@@ -353,7 +373,7 @@ static void factor_symmetric(const SymMatrix& M, int ns, int mid, cd* dinv) {
           pivot.re[(size_t)i * n2 + j] = pivot.re[(size_t)j * n2 + i];
           pivot.im[(size_t)i * n2 + j] = pivot.im[(size_t)j * n2 + i];
         }
-      split_invert(n2, pivot);
+      if (!split_invert(n2, pivot, fan)) return false;
       for (int i = 0; i < rs; ++i) {  // panel_i = -D_ik pivot^-1
         if (i == k) continue;
         std::fill(panel[i].re.begin(), panel[i].re.end(), 0.0);
@@ -401,6 +421,7 @@ static void factor_symmetric(const SymMatrix& M, int ns, int mid, cd* dinv) {
             T.im[(size_t)q * n2 + r] = B.im[(size_t)r * n2 + q];
           }
       }
+    return true;
   };
   auto pivot_block = [&](int s) {
     const int rs = rows(s);
@@ -432,22 +453,23 @@ static void factor_symmetric(const SymMatrix& M, int ns, int mid, cd* dinv) {
   for (int s = 0; s < mid; ++s) {
     pivot_block(s);
     if (s > 0) subtract(s, s - 1, Dl);
-    invert(rows(s));
+    if (!invert(rows(s))) return false;
     store(s);
     Dl = D;
   }
   for (int s = ns - 1; s > mid; --s) {
     pivot_block(s);
     if (s < ns - 1) subtract(s, s + 1, Dr);
-    invert(rows(s));
+    if (!invert(rows(s))) return false;
     store(s);
     Dr = D;
   }
   pivot_block(mid);
   if (mid > 0) subtract(mid, mid - 1, Dl);
   if (mid < ns - 1) subtract(mid, mid + 1, Dr);
-  invert(rows(mid));
+  if (!invert(rows(mid))) return false;
   store(mid);
+  return true;
 }
 
 // out_I = B_I x_I for all blocks I of all channels; 8 threads per row
@@ -978,9 +1000,13 @@ extern "C" int pp_precond_create(int nchan, int n1, int n2, int band, const doub
       for (int d = 0; d < w; ++d)
         for (int i = 0; i < n2; ++i)
           if (i + d - band >= 0 && i + d - band < n2) s2b[(size_t)d * n2 + i] = s2[(size_t)i * n2 + i + d - band];
+      std::atomic<bool> fits{true};
       each_channel([&](int c) {
         const SymMatrix M = matrix(c);
-        factor_symmetric(M, ns, mid, dinv.data() + (size_t)c * ns * m * m);
+        if (!fits || !factor_symmetric(M, ns, mid, dinv.data() + (size_t)c * ns * m * m)) {
+          fits = false;
+          return;
+        }
         for (int I = 0; I < n1; ++I)
           for (int delta = 1; delta <= band && I + delta < n1; ++delta)
             for (int d = 0; d < w; ++d)
@@ -988,30 +1014,32 @@ extern "C" int pp_precond_create(int nchan, int n1, int n2, int band, const doub
                 if (i + d - band >= 0 && i + d - band < n2)
                   pc[((((size_t)c * n1 + I) * band + delta - 1) * w + d) * n2 + i] = M.pval(I, I + delta, i, i + d - band);
       });
-      auto* p = new pp_precond();
-      try {
-        Precond& q = p->p;
-        q.nchan = nchan;
-        q.n1 = n1;
-        q.n2 = n2;
-        q.b = band;
-        q.sym = true;
-        q.ns = ns;
-        q.mid = mid;
-        q.sh = make_double2(sh.real(), sh.imag());
-        q.ss = make_double2(ss.real(), ss.imag());
-        q.dinv.upload(reinterpret_cast<const double2*>(dinv.data()), dinv.size());
-        q.pc.upload(pc.data(), pc.size());
-        q.s1.upload(s1b.data(), s1b.size());
-        q.s2.upload(s2b.data(), s2b.size());
-        sym_prepare(q);
-        PP_HIP(hipDeviceSynchronize());
-      } catch (...) {
-        delete p;
-        throw;
+      if (fits) {
+        auto* p = new pp_precond();
+        try {
+          Precond& q = p->p;
+          q.nchan = nchan;
+          q.n1 = n1;
+          q.n2 = n2;
+          q.b = band;
+          q.sym = true;
+          q.ns = ns;
+          q.mid = mid;
+          q.sh = make_double2(sh.real(), sh.imag());
+          q.ss = make_double2(ss.real(), ss.imag());
+          q.dinv.upload(reinterpret_cast<const double2*>(dinv.data()), dinv.size());
+          q.pc.upload(pc.data(), pc.size());
+          q.s1.upload(s1b.data(), s1b.size());
+          q.s2.upload(s2b.data(), s2b.size());
+          sym_prepare(q);
+          PP_HIP(hipDeviceSynchronize());
+        } catch (...) {
+          delete p;
+          throw;
+        }
+        *out = p;
+        return;
       }
-      *out = p;
-      return;
     }
     const size_t bs = (size_t)n2 * n2;
     HostFactors F;

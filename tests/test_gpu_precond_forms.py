@@ -30,7 +30,17 @@ def _pairs(n, b):
     return np.array([(i, j) for i in range(n) for j in range(max(0, i - b), min(n, i + b + 1))], dtype=np.int32)
 
 
-def _check(torch, nchan, n1, n2, b, kind, sh, ss, seed=0, before_solve=None):
+def _growth(M):
+    """The largest entry of the factors without pivoting over the largest of M: what the backward error of
+    such an elimination is proportional to."""
+    A = M.copy()
+    for k in range(len(A)):
+        A[k + 1:, k] /= A[k, k]
+        A[k + 1:, k + 1:] -= np.outer(A[k + 1:, k], A[k, k + 1:])
+    return np.abs(A).max() / np.abs(M).max()
+
+
+def _check(torch, nchan, n1, n2, b, kind, sh, ss, seed=0, before_solve=None, indefinite=False):
     from pyprop_amd import _native as N, device as D
     rng = np.random.default_rng(seed)
     S1, S2 = _band(rng, n1, b), _band(rng, n2, b)
@@ -62,7 +72,8 @@ def _check(torch, nchan, n1, n2, b, kind, sh, ss, seed=0, before_solve=None):
         M = (M + ss * np.einsum("ab,cd->acbd", S1, S2)).reshape(n1 * n2, n1 * n2)
         ref = np.linalg.solve(M, x[c].ravel())
         err = np.linalg.norm(got[c].ravel() - ref) / np.linalg.norm(ref)
-        assert err < 1e-14 * np.linalg.cond(M) * 4, (c, err)
+        bound = 4e-14 if not indefinite else 16 * 2.0 ** -53 * _growth(M)
+        assert err < bound * np.linalg.cond(M), (c, err)
 
 
 # two to ten superblocks, a short last one, each band limit (4, 6, 8) with each of its counts of 64-column tiles
@@ -95,3 +106,13 @@ def test_block_rows_beyond_the_superblock_kernel(torch):
 def test_real_scaling(torch):
     """H - sigma S with sigma below the spectrum, as the shift-invert solver asks for it."""
     _check(torch, 2, 13, 12, 4, "symmetric", 0.2, 1.5)
+
+
+# sigma inside the spectrum: H - sigma S is indefinite, real or nearly so
+@pytest.mark.parametrize("seed", range(4))
+@pytest.mark.parametrize("ss", [-0.5, 0.3, -0.1 + 1e-6j])
+@pytest.mark.parametrize("size", [(13, 13, 4), (20, 20, 5), (24, 24, 6)], ids=lambda s: "x".join(map(str, s)))
+def test_shift_inside_the_spectrum(torch, size, ss, seed):
+    """Elimination without pivoting loses digits to the growth of its factors, and explicit inverses of
+    whole superblocks more than that: such matrices are factorized as a block LU."""
+    _check(torch, 1, *size, "symmetric", 1.0, ss, seed=seed, indefinite=True)
