@@ -236,13 +236,14 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
   };
   // (by components: an array of whole values copied from memory and on to LDS was kept in scratch memory,
   // 23 us instead of 7 for 8 x 40 x 96 with 3 diagonals)
+  typedef decltype(C::x) Pair __attribute__((ext_vector_type(2)));
   // source values of a tuple, and the bands of its row r per lane (lanes past the fibre repeat its last row)
   auto load_x = [&](const int4& tp, C (&x)[NR]) {
     const C* xp = a.src + (long long)tp.x * n;
     for_rows<NR>([&](auto r) {
-      const C& v = xp[min(lane + 64 * r, n - 1)];
-      x[r].x = v.x;
-      x[r].y = v.y;
+      const Pair v = *reinterpret_cast<const Pair*>(xp + min(lane + 64 * r, n - 1));
+      x[r].x = v[0];
+      x[r].y = v[1];
     });
   };
   auto load_row = [&](const int4& tp, int r, V (&v)[BW]) {
@@ -269,10 +270,7 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
   };
   auto window = [&](const C (&x)[NR]) {
     for_rows<NR>([&](auto r) {
-      if (lane + 64 * r < n) {
-        xw[HB + lane + 64 * r].x = x[r].x;
-        xw[HB + lane + 64 * r].y = x[r].y;
-      }
+      if (lane + 64 * r < n) *reinterpret_cast<Pair*>(xw + HB + lane + 64 * r) = Pair{x[r].x, x[r].y};
     });
     wave_sync();
   };
