@@ -1,11 +1,12 @@
 // The S-metric inner product without any device allocation, for callers that cannot
 // allocate (code under stream capture, tight serving loops, harnesses that forbid hipMalloc).
 //
-// pp_repr_inner_product allocates its reduction partials on every call and grows each
-// overlap factor's out-of-place pass buffer on demand.  pp_repr_inner_product_noalloc runs
-// the same kernels (the copy of b, the S passes of every non-orthogonal rank, the two-stage
-// deterministic dot), so its result is bitwise the same, but every intermediate lives in
-// one file-scope device array, `scratch`:
+// pp_repr_inner_product allocates its reduction partials on every call and, where the S
+// passes do not run on tiles (overlap.hip), grows each overlap factor's out-of-place pass
+// buffer on demand.  pp_repr_inner_product_noalloc copies b and multiplies the copy by S in
+// place, where the other reads b itself; the S passes of every non-orthogonal rank and the
+// two-stage deterministic dot are the same kernels with the same arithmetic, so its result
+// is bitwise the same, but every intermediate lives in one file-scope device array, `scratch`:
 //
 //   [0, kMaxElements)                 copy of b, multiplied by S in place
 //   [kMaxElements, 2 kMaxElements)    out-of-place buffer of the S passes

@@ -12,20 +12,26 @@
 // owns one destination fibre, so no atomics are needed and the summation order is fixed
 // (deterministic).  Its four waves split the fibre's tuple list in four contiguous parts
 // whose partial sums are added in order at the end.  Workgroups are launched in order of
-// decreasing tuple count (longest first) to balance the tail.
+// decreasing tuple count (longest first) to balance the tail, those of compact plans in
+// an order by XCD (xcd_order).
 //
 // Innermost rank:
 //  * banded storages (BandNH = zgbmv, Band = zhbmv) are re-laid out once into
 //    diagonal-major form D[fibre][d][i] = A(i, i + d - hb): lane i streams row i with
 //    fully coalesced loads (consecutive lanes read consecutive addresses), the source
 //    window is staged in LDS per wave.  If every imaginary part is zero the diagonals are
-//    stored as float64 (8 B/element instead of 16).  This path is HBM-bound.
+//    stored as float64 (8 B/element instead of 16).  Streamed in this form the path is
+//    HBM-bound.
 //    Real potentials are then stored once where they repeat (compact_term): a term whose bands
 //    are all symmetric keeps the diagonals d >= hb only, row i of a lower diagonal being read at
 //    row i - (hb - d) of its mirror image; fibres that are equal bit for bit are kept once.
 //    Potentials of this kind repeat a lot: (i1, j1) and (j1, i1) give the same band, and so do
-//    the angular pairs (c, c') and (c', c).  Helium (42 channels x 60 x 60): 0.49 GB kept of 2.65.
-//    The sums and their order do not change.
+//    most angular pairs (c, c') and (c', c).  What differs in its last bit is kept apart: helium
+//    (42 channels x 60 x 60, 2.65 GB) keeps 0.49 GB when generated from the grid, 1.09 GB when
+//    expanded from the host's radial factors, whose 1/r12 bands are not symmetric to the bit.
+//    Where mirror images are read the sums and their order do not change.  Where they are not
+//    (all terms symmetric, n <= 64), a lower diagonal's product is v (s x) instead of s (v x) and
+//    is added to its row at the end: other roundings, of the same number of operations.
 //  * all other storages go through a generic per-row entry list (CSR) over the
 //    reference layout; correct for every storage, not tuned.
 #include <hip/hip_runtime.h>
@@ -194,8 +200,9 @@ __device__ __forceinline__ void for_rows(F&& f) {
 // COMPACT: kMixed, some term is stored compactly; kSymmetric, all are and keep half the diagonals (the
 // offsets then are the same for every tuple).  Their values are read again soon (as a mirror image, or by
 // another fibre), so they are left in the caches instead of streamed past them.  Helium's full H in
-// FP64: 428 us streaming every fibre (HBM), 172 us, bound by the L1's rate of 8-byte loads: 251 with the
-// mirror images read as well (16 clocks of a CU per load instruction).
+// FP64: 428 us streaming every fibre (HBM); 172 us, in which the 0.49 GB stored come into the XCDs' L2s 2.5
+// times each, 1.24 GB at 7.2 TB/s, while the L1s' 8-byte loads (16 clocks of a CU each) take half the
+// clocks; 251 with the mirror images read as well.
 template <class V, class C, int BW, int NR, int COMPACT>
 __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
   constexpr int HB = (BW - 1) / 2;
