@@ -75,6 +75,21 @@ def matvec_input(torch, repr_, shape, seed=2024):
     return w
 
 
+def potgen_bytes(shape, grid, terms):
+    """Bytes that generating a potential of `shape` (pairs per rank) moves, for grid terms of
+    `terms` radial functions each on a `grid` of points per radial rank.  The grid functions are
+    evaluated where they are projected; the projections onto the last rank are written and read,
+    one per angular pair or, where that is less work (`project_terms` in potgen.hip), one per
+    radial function with the projected functions written and read too; the complex result is
+    written, and read as well from the second grid term on."""
+    P0, P1, P2 = shape
+    Q1 = grid[0]
+    nbytes = (2 * len(terms) - 1) * 16 * P0 * P1 * P2
+    for T in terms:
+        nbytes += 2 * 8 * P2 * (T * (Q1 + P1) if T * (Q1 + P1) <= P0 * Q1 else P0 * Q1)
+    return nbytes
+
+
 def time_potgen(torch, sysm, reps=3):
     """Device generation (grid evaluation + two B-spline projections) of every helium
     potential: wall time per potential with HIP events on torch's current stream (the
@@ -93,13 +108,9 @@ def time_potgen(torch, sysm, reps=3):
         ev1.record()
         torch.cuda.synchronize()
         ms = ev0.elapsed_time(ev1) / reps
-        P0, P1, P2 = p.shape
-        Q1, Q2 = (g.basis.grid.size for g in p.geometries[1:])
-        terms = len(p.grid_terms)
-        # per grid term: grid write + read, intermediate (P0, Q1, P2) write + read, complex result
-        # write (read + write when accumulating)
-        nbytes = terms * (2 * 8 * P0 * Q1 * Q2 + 2 * 8 * P0 * Q1 * P2) + (2 * terms - 1) * 16 * P0 * P1 * P2
-        out[p.name.split("+")[0]] = {"ms": ms, "shape": [P0, P1, P2], "grid_terms": terms,
+        nbytes = potgen_bytes(p.shape, [g.basis.grid.size for g in p.geometries[1:]],
+                              [len(t.coeffs) for t in p.grid_terms])
+        out[p.name.split("+")[0]] = {"ms": ms, "shape": list(p.shape), "grid_terms": len(p.grid_terms),
                                      "bytes": nbytes, "GB_per_s": nbytes / ms / 1e6}
         log("device generation %-40s %s: %.2f ms, %.1f GB/s" % (p.name[:40], p.shape, ms, nbytes / ms / 1e6))
         torch.cuda.empty_cache()
@@ -107,8 +118,9 @@ def time_potgen(torch, sysm, reps=3):
 
 
 def profiled_traffic():
-    """HBM bytes per launch of the fused multiply from the committed rocprofv3 counter
-    summary (FETCH_SIZE + WRITE_SIZE, copy-calibrated), or None."""
+    """Bytes that one launch of the fused multiply, of compactly stored potentials, moves beyond
+    the L2 caches, from the committed rocprofv3 counter summary (FETCH_SIZE + WRITE_SIZE,
+    copy-calibrated), or None."""
     path = ROOT / "profiles" / "tp_dia_kernel_helium_fp64_matvec.md"
     if not path.exists():
         return None
@@ -779,6 +791,7 @@ def main():
     for v in runs.values():
         v.pop("check", None)
 
+    traffic = profiled_traffic()
     out = {
         "metric": "CN steps/s, helium rank-3: learned+FP32 vs plain FP64 GPU at 1e-8 err; GB/s",
         "value": lrn["steps_per_s"],
@@ -827,7 +840,8 @@ def main():
                    "potential_generation": potgen,
                    "cpu_baseline_single_thread": cpu1},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": profiled_traffic(),
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
+                     "traffic_GBps": traffic / t_mv / 1e9 if traffic else None,
                      "traffic_source": "profiles/tp_dia_kernel_helium_fp64_matvec.md (rocprofv3 FETCH_SIZE + "
                                        "WRITE_SIZE, scaled by a 1 GiB copy)",
                      "kernel": "tp_dia_kernel (fused H0+R12+dipole FP64 multiply)", "ms": t_mv * 1e3,

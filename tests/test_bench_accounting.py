@@ -38,3 +38,11 @@ def test_issued_mfma_matches_hardware_counts(radial, counted, angular):
     issued, useful = bench.factored_flops(_Helium(radial, angular), 42, 60, 64)
     assert issued == (counted + (0 if angular.startswith("sparse") else 259200)) * 2048
     assert 0 < useful < issued
+
+
+def test_generation_bytes_follow_the_form_that_runs():
+    """Helium's 1/r12 (394 angular pairs, 11 multipole terms on 392 points): its terms are projected, not
+    its pairs; two pairs of two terms are projected pair by pair."""
+    result = 16 * 394 * 738 * 780
+    assert bench.potgen_bytes((394, 738, 780), (392, 392), [11]) == result + 16 * 780 * 11 * (392 + 738)
+    assert bench.potgen_bytes((2, 20, 30), (40, 40), [2, 2]) == 3 * 16 * 2 * 20 * 30 + 2 * 16 * 30 * 2 * 40
