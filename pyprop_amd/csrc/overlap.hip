@@ -335,10 +335,10 @@ static bool overlap_tile(const OverlapFactor& ov, int op, bool conj, long long p
   // coefficients are read once for FT fibres.  A solve's are as wide as leaves 64 KB of LDS for the
   // partial sums; a multiply's have four fibres, as narrower ones of a rank that is not the last take
   // less than 64 bytes of a row and a cache line then goes to several XCDs
-  const bool few = fibres <= (solve || post == 1 ? 512 : 128);
+  const bool few = fibres <= (solve || post == 1 || n <= 160 ? 512 : 128);
   const int ft = few ? 1 : post == 2 ? 2 : solve && n <= 64 ? 8 : n <= 160 || (!solve && post > 1) ? 4 : n <= 320 ? 2 : 1;
   const int parts = solve ? std::max(1, std::min(ft >= 4 ? 4 : 8, 16 / groups)) : second < 0 ? 0 : 1;
-  const int threads = solve ? 64 * groups * parts : n * ft <= 640 ? 256 : 1024;
+  const int threads = solve ? 64 * groups * parts : std::max(256, std::min(1024, (n * ft + 63) / 64 * 64));
   const size_t lds = tile_lds(n, ft, parts, solve ? -1 : ov.sd);
   const long long blocks = tile_count(pre, post, ft);
   if (!launchable(blocks, threads)) return false;
@@ -515,22 +515,22 @@ static void launch_window(int op, bool conj, const double* u, int n, long long p
 // superdiagonals:
 //   fibres x rows   2520 x 60  20000 x 60  80000 x 60  20000 x 160  2520 x 200  20000 x 200  2520 x 512
 //   S^-1              46 / 9     48 / 29     91 / 101    137 / 132    150 / 35    175 / 241    406 / 311
-//     (two superdiagonals, 20000 x 160: 108 / 131)
+//     (two superdiagonals, 20000 x 160: 108 / 131; 10000 x 320: 272 / 241)
 //   U^-1              35 / 11    36 / 15     51 / 45     110 / 57     114 / 45    139 / 181    287 / 134
 //   U^-H              22 / 11    21 / 15     48 / 45      61 / 58      69 / 45     78 / 180    173 / 135
-// and 20000 x 512 up to five times slower on tiles.  Below 16 rows both take the launch.
+// and 20000 x 512 up to five times slower on tiles.
 // The multiplies have no chain, and spare a pass over memory on tiles.
 static bool in_tiles(const OverlapFactor& ov, int op, bool conj, long long fibres) {
   const int n = ov.n;
   if (n > kTileRows) return false;
   const long long values = fibres * n;
   if (op == PP_OVERLAP_SOLVE)
-    return n >= 16 && fibres <= 32768 && values <= (n <= 160 && ov.sd >= 6 ? 3200000 : n <= 320 ? 2500000 : 1300000);
+    return fibres <= 32768 && values <= (n > 320 ? 1300000 : n > 256 || (n <= 160 && ov.sd >= 6) ? 3200000 : 2500000);
   if (op == PP_OVERLAP_SQRT_SOLVE) {
-    if (ov.sd < 1 || ov.sd > 8 || n < 16) return false;
+    if (ov.sd < 1 || ov.sd > 8) return false;
     if (n <= 160) return fibres <= 32768 && (!conj || values <= 3200000);
     const long long work = values * (std::max(ov.sd, 6) + 2);
-    return conj ? fibres <= 4000 && work <= 8 * 1300000 : work <= 8 * 2600000;
+    return conj ? fibres <= 4000 && work <= 8 * 1300000 : work <= 8 * (n > 256 ? 3300000 : 2600000);
   }
   return ov.sd <= 8;
 }
