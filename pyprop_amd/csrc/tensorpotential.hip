@@ -241,27 +241,38 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
   auto tuple = [&](int l) {
     return make_int4(from_lane(tup_l.x, l), from_lane(tup_l.y, l), from_lane(tup_l.z, l), 0);
   };
-  // (by components: an array of whole values copied from memory and on to LDS was kept in scratch memory,
-  // 23 us instead of 7 for 8 x 40 x 96 with 3 diagonals)
+  // Source values of a tuple, and the bands of its row r per lane (lanes past the fibre repeat its last
+  // row).  Several rows through a descriptor and by components: an array of whole values copied from memory
+  // and on to LDS was kept in scratch memory, 23 us instead of 7 for 8 x 40 x 96 with 3 diagonals.  One row
+  // plainly (13 x 30 x 30: 13.1 us, 13.6 through a descriptor).
   typedef decltype(C::x) Pair __attribute__((ext_vector_type(2)));
-  // source values of a tuple, and the bands of its row r per lane (lanes past the fibre repeat its last row)
   auto load_x = [&](const int4& tp, C (&x)[NR]) {
     const C* xp = a.src + (long long)tp.x * n;
-    for_rows<NR>([&](auto r) {
-      const Pair v = *reinterpret_cast<const Pair*>(xp + min(lane + 64 * r, n - 1));
-      x[r].x = v[0];
-      x[r].y = v[1];
-    });
+    if constexpr (NR == 1) {
+      x[0] = xp[min(lane, n - 1)];
+    } else {
+      const __amdgpu_buffer_rsrc_t fibre =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<C*>(xp), (short)0, n * (int)sizeof(C), 0x00020000);
+      for_rows<NR>([&](auto r) {
+        const Pair v = ld_band<Pair, true>(fibre, min(lane + 64 * r, n - 1) * (int)sizeof(C), 0);
+        x[r].x = v[0];
+        x[r].y = v[1];
+      });
+    }
   };
-  auto load_row = [&](const int4& tp, int r, V (&v)[BW]) {
+  auto is_sym = [&](const int4& tp) {
+    return COMPACT == kSymmetric || (COMPACT == kMixed && (a.sym >> (tp.z >> 1) & 1));
+  };
+  auto bands = [&](const int4& tp) {  // the tuple's potential fibre
     const int term = tp.z >> 1;
-    const bool sym = COMPACT == kSymmetric || (COMPACT == kMixed && (a.sym >> term & 1));
     const unsigned long long base = (unsigned)from_lane((int)(dia_l & 0xffffffffu), term) |
                                     (unsigned long long)(unsigned)from_lane((int)(dia_l >> 32), term) << 32;
-    const int fibre = (sym ? HB + 1 : BW) * n;  // stored values of a potential fibre
-    const __amdgpu_buffer_rsrc_t band = __builtin_amdgcn_make_buffer_rsrc(
+    const int fibre = (is_sym(tp) ? HB + 1 : BW) * n;  // stored values of a potential fibre
+    return __builtin_amdgcn_make_buffer_rsrc(
         reinterpret_cast<void*>(base + (unsigned long long)tp.y * fibre * sizeof(V)), (short)0,
         fibre * (int)sizeof(V), 0x00020000);
+  };
+  auto load_row = [&](__amdgpu_buffer_rsrc_t band, bool sym, int r, V (&v)[BW]) {
     const int i = lane + 64 * r;
 #pragma unroll
     for (int k = 0; k <= HB; ++k)
@@ -276,9 +287,13 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
       }
   };
   auto window = [&](const C (&x)[NR]) {
-    for_rows<NR>([&](auto r) {
-      if (lane + 64 * r < n) *reinterpret_cast<Pair*>(xw + HB + lane + 64 * r) = Pair{x[r].x, x[r].y};
-    });
+    if constexpr (NR == 1) {
+      if (lane < n) xw[HB + lane] = x[0];
+    } else {
+      for_rows<NR>([&](auto r) {
+        if (lane + 64 * r < n) *reinterpret_cast<Pair*>(xw + HB + lane + 64 * r) = Pair{x[r].x, x[r].y};
+      });
+    }
     wave_sync();
   };
   auto use_row = [&](const int4& tp, auto r, const C& x, const V (&v)[BW]) {
@@ -316,8 +331,9 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
       // the next tuple's loads are issued before the current one is used: a wave waits for memory about
       // half as often, for one more set of registers
       auto load = [&](const int4& tp, C (&x)[NR], V (&v)[NR][BW]) {
+        const __amdgpu_buffer_rsrc_t band = bands(tp);
         load_x(tp, x);
-        for_rows<NR>([&](auto r) { load_row(tp, r, v[r]); });
+        for_rows<NR>([&](auto r) { load_row(band, is_sym(tp), r, v[r]); });
       };
       auto use = [&](const int4& tp, const C (&x)[NR], const V (&v)[NR][BW]) {
         window(x);
@@ -346,14 +362,15 @@ __global__ __launch_bounds__(256) void tp_dia_kernel(DiaArgs<C> a) {
       for (int l = 0; l <= last; ++l) {
         const int4 tp = tuple(l);
         C x[NR];
+        const __amdgpu_buffer_rsrc_t band = bands(tp);
         load_x(tp, x);
         V v[kAhead + 1][BW];
-        load_row(tp, 0, v[0]);
+        load_row(band, is_sym(tp), 0, v[0]);
         window(x);
         for_rows<NR>([&](auto r) {
           constexpr int R = decltype(r)::value;
-          if constexpr (kAhead == 1 && R + 1 < NR) load_row(tp, R + 1, v[(R + 1) & 1]);
-          if constexpr (kAhead == 0 && R > 0) load_row(tp, R, v[0]);
+          if constexpr (kAhead == 1 && R + 1 < NR) load_row(band, is_sym(tp), R + 1, v[(R + 1) & 1]);
+          if constexpr (kAhead == 0 && R > 0) load_row(band, is_sym(tp), R, v[0]);
           use_row(tp, r, x[r], v[R & kAhead]);
         });
         wave_sync();
